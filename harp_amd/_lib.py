@@ -51,10 +51,21 @@ ABI_PROTOTYPES = {
         [_p, _i64p, _pp, _pp, _i64p, _i, _i32p, _p, _i64p, _p, _i, _p,
          _i, _i, _i, _i, _i, _i, ctypes.c_float, _p, _sz, _p],
     ),
+    "harp_ra_forward_rounded": (
+        _i,
+        [_p, _i64p, _pp, _pp, _i64p, _i, _i32p, _p, _i64p, _p, _i64p, _p, _i, _p,
+         _i, _i, _i, _i, _i, _i, ctypes.c_float, _p, _sz, _p],
+    ),
     "harp_ra_backward": (
         _i,
         [_p, _i64p, _p, _i64p, _i, _pp, _pp, _i64p, _pp, _pp, _i64p, _i,
          _i, _i32p, _p, _i64p, _p, _i, _p, _p,
+         _i, _i, _i, _i, _i, _i, ctypes.c_float, _p, _sz, _p],
+    ),
+    "harp_ra_backward_from_out": (
+        _i,
+        [_p, _i64p, _p, _i64p, _i, _pp, _pp, _i64p, _pp, _pp, _i64p, _i,
+         _i, _i32p, _p, _i64p, _p, _i, _p, _p, _i64p,
          _i, _i, _i, _i, _i, _i, ctypes.c_float, _p, _sz, _p],
     ),
     "harp_ra_delta": (_i, [_p, _i64p, _p, _i64p, _p, _i, _i, _i, _i, _p]),

@@ -74,6 +74,7 @@ __global__ __launch_bounds__(64 * kAsmWaves, 1) void dq_asm_kernel(BwdParams p) 
   // registers: one row per lane straight from global memory took twice as
   // long per block.
   v32i q0, q1, g0, g1;
+  float dsum[16];  // without p.delta: dsum[0] = D of the wave's row 4 (lane % 16) + lane / 16
   {
     const int r0 = qt * kAsmRows;
     const rsrc_t rq = rows_rsrc(p.q + (int64_t)b * p.sqb + (int64_t)h * p.sqh, p.sqt, r0, p.T - r0);
@@ -85,8 +86,52 @@ __global__ __launch_bounds__(64 * kAsmWaves, 1) void dq_asm_kernel(BwdParams p) 
       lds_dma_b128(rq, lds0 + inst * 1024, (uint32_t)(row * p.sqt * 2) + chunk);
       lds_dma_b128(rg, lds0 + 65536 + inst * 1024, (uint32_t)(row * p.sdt * 2) + chunk);
     }
+    // D = rowsum(dO O) of the wave's 64 rows, 16 lanes x 8 elements per row,
+    // four rows a step: O's rows are requested here, beside the copies, and
+    // dO's are read back from LDS, so the block pays no launch and no second
+    // read of dO for it (delta_kernel took 4 us at 30 heads x 256 rows, 24 us
+    // at 24 x 8192).  One forward + backward at 30 x 256 rows, 8 chunks: 128
+    // us before, 102 with D, the cast and the fill of m in these kernels
+    const int sub = lane & 15, rr = lane >> 4;
+    f32x4u ox[16], oy[16];
+    if (!p.delta) {
+      const float* ob = p.out + (int64_t)b * p.sob + (int64_t)h * p.soh + sub * 8;
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        const int qi = r0 + wave * 64 + 4 * i + rr;
+        const float* orow = ob + (int64_t)(qi < p.T ? qi : r0) * p.sot;  // past T: any row, its dO is zero
+        ox[i] = *(const f32x4u*)orow;
+        oy[i] = *(const f32x4u*)(orow + 4);
+      }
+    }
     wait_lds_loads();
     __syncthreads();
+    if (!p.delta) {
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        const int row = wave * 64 + 4 * i + rr;
+        const bf16x8 x = *(const bf16x8*)(lds + 65536 + row * 256 + ((sub ^ swz(row)) << 4));
+        float acc = 0.f;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          acc = __builtin_fmaf((float)x[j], ox[i][j], acc);
+          acc = __builtin_fmaf((float)x[j + 4], oy[i][j], acc);
+        }
+        dsum[i] = acc;
+      }
+      // 16 sums over the 16 lanes of a row at once: each exchange halves the
+      // values a lane still holds (15 exchanges, not 64), lane `sub` ends
+      // with the sum of step i = sub
+#pragma unroll
+      for (int w = 8; w >= 1; w >>= 1) {
+        const bool up = (sub & w) != 0;
+#pragma unroll
+        for (int i = 0; i < w; ++i) {
+          const float keep = up ? dsum[i + w] : dsum[i], give = up ? dsum[i] : dsum[i + w];
+          dsum[i] = keep + __shfl_xor(give, w, 16);
+        }
+      }
+    }
 #pragma unroll
     for (int qg = 0; qg < 2; ++qg) {
       const int row = wave * 64 + qg * 32 + l32;
@@ -121,7 +166,9 @@ __global__ __launch_bounds__(64 * kAsmWaves, 1) void dq_asm_kernel(BwdParams p) 
       const bool ok = qi < p.T;
       const int64_t si = ((int64_t)b * p.H + h) * p.T + (ok ? qi : 0);
       st0[qg] = ok ? bwd_stat_lse(p, si) : 0.f;
-      st1[qg] = ok ? -p.delta[si] : 0.f;
+      const int row = qg * 32 + l32;  // of the wave: step row / 4, lane group row % 4
+      const float d = p.delta ? p.delta[si] : __shfl(dsum[0], (row & 3) * 16 + (row >> 2));
+      st1[qg] = ok ? -d : 0.f;
       if (ok && g == 0 && sp.index == 0) {
         p.stats[si] = st0[qg];
         p.stats[nrows + si] = st1[qg];

@@ -104,6 +104,18 @@ int check_out_view(const void* p, const int64_t* s, int B, int H, int rows, int 
   return HARP_RA_OK;
 }
 
+// The rounded output: a non-overlapping view written four elements (8 bytes)
+// at a time.
+int check_rounded_out(const void* p, const int64_t* s, int B, int H, int rows, int D) {
+  if (int rc = check_out_view(p, s, B, H, rows, D, "out_rounded")) return rc;
+  const int64_t ext[3] = {B, H, rows};
+  for (int i = 0; i < 3; ++i)
+    if (ext[i] > 1 && s[i] % 4 != 0)
+      return fail(HARP_RA_EINVAL, "out_rounded stride[%d]=%lld must be a multiple of 4 elements", i, (long long)s[i]);
+  if ((reinterpret_cast<uintptr_t>(p) & 7u) != 0) return fail(HARP_RA_EINVAL, "out_rounded must be 8-byte aligned");
+  return HARP_RA_OK;
+}
+
 // Streamed operands are read through 32-bit buffer offsets: every [rows][D]
 // view the kernels walk (one (b, h) of a chunk, of q or of grad_out) must
 // span less than 2^31 bytes, counted over at least 128 rows: the copies of a
@@ -300,63 +312,13 @@ int launched(hipError_t e, const char* what) {
   return HARP_RA_OK;
 }
 
-}  // namespace
-
-extern "C" {
-
-const char* harp_ra_last_error(void) { return g_last_error.c_str(); }
-
-const char* harp_ra_version(void) { return "harp_ra 0.1.0 (gfx950)"; }
-
-int harp_ra_timing_enable(int enable) {
-  timing().on = (enable != 0);
-  return ok();
-}
-
-int harp_ra_timing_read(double* ms, int* launches, int n_kinds) {
-  if (!ms || !launches || n_kinds < 1) return fail(HARP_RA_EINVAL, "timing_read needs output arrays");
-  for (int i = 0; i < n_kinds; ++i) {
-    ms[i] = 0.0;
-    launches[i] = 0;
-  }
-  Timing& t = timing();
-  int rc = HARP_RA_OK;
-  for (auto& r : t.recs) {
-    float e = 0.f;
-    if (hipEventElapsedTime(&e, r.a, r.b) != hipSuccess) rc = HARP_RA_ELAUNCH;
-    if (r.kind < n_kinds) {
-      ms[r.kind] += e;
-      launches[r.kind] += 1;
-    }
-    t.pool.push_back(r.a);
-    t.pool.push_back(r.b);
-  }
-  t.recs.clear();
-  if (rc) return fail(rc, "hipEventElapsedTime failed (were the streams synchronised?)");
-  return ok();
-}
-
-size_t harp_ra_forward_workspace_bytes(int batch, int h_num, int t_num, int h_len, int sp_size, int kv_chunk_len,
-                                       const int32_t* kv_valid_lens) {
-  Geometry g;
-  if (check_dims(batch, h_num, t_num, h_len) != HARP_RA_OK) return SIZE_MAX;
-  if (make_geometry(sp_size, kv_chunk_len, kv_valid_lens, &g) != HARP_RA_OK) return SIZE_MAX;
-  return fwd_ws(batch, h_num, t_num, h_len, g);
-}
-
-size_t harp_ra_backward_workspace_bytes(int batch, int h_num, int t_num, int h_len, int sp_size, int kv_chunk_len,
-                                        const int32_t* kv_valid_lens) {
-  Geometry g;
-  if (check_dims(batch, h_num, t_num, h_len) != HARP_RA_OK) return SIZE_MAX;
-  if (make_geometry(sp_size, kv_chunk_len, kv_valid_lens, &g) != HARP_RA_OK) return SIZE_MAX;
-  return bwd_ws(batch, h_num, t_num, h_len, g);
-}
-
-int harp_ra_forward(const void* q, const int64_t* q_strides, const void* const* k_chunks,
-                    const void* const* v_chunks, const int64_t* kv_strides, int kv_chunk_len,
-                    const int32_t* kv_valid_lens, float* out, const int64_t* out_strides, void* m_i, int m_i_dtype,
-                    float* l_i, int batch, int h_num, int t_num, int h_len, int sp_size, int ring_rank, float scale,
-                    void* workspace, size_t workspace_bytes, void* stream) {
+// harp_ra_forward and harp_ra_forward_rounded: `out_rounded` (may be NULL)
+// receives O in bf16; `out` may be NULL only when it is given.
+int forward_impl(const void* q, const int64_t* q_strides, const void* const* k_chunks, const void* const* v_chunks,
+                 const int64_t* kv_strides, int kv_chunk_len, const int32_t* kv_valid_lens, float* out,
+                 const int64_t* out_strides, void* out_rounded, const int64_t* rounded_strides, void* m_i,
+                 int m_i_dtype, float* l_i, int batch, int h_num, int t_num, int h_len, int sp_size, int ring_rank,
+                 float scale, void* workspace, size_t workspace_bytes, void* stream) {
   int rc;
   if ((rc = check_dims(batch, h_num, t_num, h_len))) return rc;
   Geometry g;
@@ -370,7 +332,10 @@ int harp_ra_forward(const void* q, const int64_t* q_strides, const void* const* 
     if ((rc = check_bf16_view(k_chunks[c], kv_strides, h_len, "k chunk"))) return rc;
     if ((rc = check_bf16_view(v_chunks[c], kv_strides, h_len, "v chunk"))) return rc;
   }
-  if ((rc = check_out_view(out, out_strides, batch, h_num, t_num, h_len, "out"))) return rc;
+  if (out || !out_rounded)
+    if ((rc = check_out_view(out, out_strides, batch, h_num, t_num, h_len, "out"))) return rc;
+  if (out_rounded)
+    if ((rc = check_rounded_out(out_rounded, rounded_strides, batch, h_num, t_num, h_len))) return rc;
   if ((rc = check_extent(kv_chunk_len, kv_strides, "k/v chunk"))) return rc;
   if (!m_i || !l_i) return fail(HARP_RA_EINVAL, "m_i / l_i are NULL");
   if (m_i_dtype != HARP_RA_F32 && m_i_dtype != HARP_RA_BF16) return fail(HARP_RA_EINVAL, "m_i_dtype must be F32 or BF16");
@@ -389,9 +354,17 @@ int harp_ra_forward(const void* q, const int64_t* q_strides, const void* const* 
   p.skh = kv_strides[1];
   p.skt = kv_strides[2];
   p.out = out;
-  p.sob = out_strides[0];
-  p.soh = out_strides[1];
-  p.sot = out_strides[2];
+  if (out) {
+    p.sob = out_strides[0];
+    p.soh = out_strides[1];
+    p.sot = out_strides[2];
+  }
+  if (out_rounded) {
+    p.outb = static_cast<bf16*>(out_rounded);
+    p.sbb = rounded_strides[0];
+    p.sbh = rounded_strides[1];
+    p.sbt = rounded_strides[2];
+  }
   p.m = m_i;
   p.m_bf16 = (m_i_dtype == HARP_RA_BF16);
   p.l = l_i;
@@ -422,6 +395,11 @@ int harp_ra_forward(const void* q, const int64_t* q_strides, const void* const* 
     mp.sob = p.sob;
     mp.soh = p.soh;
     mp.sot = p.sot;
+    mp.outb = p.outb;
+    mp.sbb = p.sbb;
+    mp.sbh = p.sbh;
+    mp.sbt = p.sbt;
+    p.outb = nullptr;
     mp.m = m_i;
     mp.m_bf16 = p.m_bf16;
     mp.l = l_i;
@@ -447,41 +425,15 @@ int harp_ra_forward(const void* q, const int64_t* q_strides, const void* const* 
   return ok();
 }
 
-int harp_ra_delta(const void* grad_out, const int64_t* do_strides, const float* out, const int64_t* out_strides,
-                  float* delta, int batch, int h_num, int t_num, int h_len, void* stream) {
-  int rc;
-  if ((rc = check_dims(batch, h_num, t_num, h_len))) return rc;
-  if ((rc = check_bf16_view(grad_out, do_strides, h_len, "grad_out"))) return rc;
-  if ((rc = check_plain_view(out, out_strides, "out"))) return rc;
-  if (!delta) return fail(HARP_RA_EINVAL, "delta is NULL");
-  DeltaParams p;
-  p.dout = static_cast<const bf16*>(grad_out);
-  p.sdb = do_strides[0];
-  p.sdh = do_strides[1];
-  p.sdt = do_strides[2];
-  p.out = out;
-  p.sob = out_strides[0];
-  p.soh = out_strides[1];
-  p.sot = out_strides[2];
-  p.delta = delta;
-  p.B = batch;
-  p.H = h_num;
-  p.T = t_num;
-  p.D = h_len;
-  {
-    TimedLaunch tl(HARP_RA_KERNEL_DELTA, static_cast<hipStream_t>(stream));
-    if ((rc = launched(launch_delta(p, static_cast<hipStream_t>(stream)), "delta"))) return rc;
-  }
-  return ok();
-}
-
-int harp_ra_backward(const void* q, const int64_t* q_strides, void* grad_q, const int64_t* dq_strides, int dq_dtype,
-                     const void* const* k_chunks, const void* const* v_chunks, const int64_t* kv_strides,
-                     void* const* dk_chunks, void* const* dv_chunks, const int64_t* dkv_strides, int dkv_dtype,
-                     int kv_chunk_len, const int32_t* kv_valid_lens, const void* grad_out, const int64_t* do_strides,
-                     const void* m_i, int m_i_dtype, const float* l_i, const float* delta, int batch, int h_num,
-                     int t_num, int h_len, int sp_size, int ring_rank, float scale, void* workspace,
-                     size_t workspace_bytes, void* stream) {
+// harp_ra_backward (delta given) and harp_ra_backward_from_out (delta NULL:
+// the dQ kernel forms it from grad_out and the forward's fp32 out).
+int backward_impl(const void* q, const int64_t* q_strides, void* grad_q, const int64_t* dq_strides, int dq_dtype,
+                  const void* const* k_chunks, const void* const* v_chunks, const int64_t* kv_strides,
+                  void* const* dk_chunks, void* const* dv_chunks, const int64_t* dkv_strides, int dkv_dtype,
+                  int kv_chunk_len, const int32_t* kv_valid_lens, const void* grad_out, const int64_t* do_strides,
+                  const void* m_i, int m_i_dtype, const float* l_i, const float* delta, const float* out,
+                  const int64_t* out_strides, int batch, int h_num, int t_num, int h_len, int sp_size, int ring_rank,
+                  float scale, void* workspace, size_t workspace_bytes, void* stream) {
   int rc;
   if ((rc = check_dims(batch, h_num, t_num, h_len))) return rc;
   Geometry g;
@@ -526,7 +478,8 @@ int harp_ra_backward(const void* q, const int64_t* q_strides, void* grad_q, cons
   if ((rc = check_extent(kv_chunk_len, kv_strides, "k/v chunk"))) return rc;
   if ((rc = check_extent(t_num, q_strides, "q"))) return rc;
   if ((rc = check_extent(t_num, do_strides, "grad_out"))) return rc;
-  if (!m_i || !l_i || !delta) return fail(HARP_RA_EINVAL, "m_i / l_i / delta are NULL");
+  if (!m_i || !l_i) return fail(HARP_RA_EINVAL, "m_i / l_i / delta are NULL");
+  if (!delta && (rc = check_plain_view(out, out_strides, "out"))) return rc;
   if (m_i_dtype != HARP_RA_F32 && m_i_dtype != HARP_RA_BF16) return fail(HARP_RA_EINVAL, "m_i_dtype must be F32 or BF16");
 
   const BwdLayout wl = bwd_layout(batch, h_num, t_num, h_len, g);
@@ -559,6 +512,12 @@ int harp_ra_backward(const void* q, const int64_t* q_strides, void* grad_q, cons
   p.m_bf16 = (m_i_dtype == HARP_RA_BF16);
   p.l = l_i;
   p.delta = delta;
+  if (!delta) {
+    p.out = out;
+    p.sob = out_strides[0];
+    p.soh = out_strides[1];
+    p.sot = out_strides[2];
+  }
   p.B = batch;
   p.H = h_num;
   p.T = t_num;
@@ -619,6 +578,136 @@ int harp_ra_backward(const void* q, const int64_t* q_strides, void* grad_q, cons
     if ((rc = launched(launch_dkdv(pk, st), "dK/dV"))) return rc;
   }
   return ok();
+}
+
+}  // namespace
+
+extern "C" {
+
+const char* harp_ra_last_error(void) { return g_last_error.c_str(); }
+
+const char* harp_ra_version(void) { return "harp_ra 0.1.0 (gfx950)"; }
+
+int harp_ra_timing_enable(int enable) {
+  timing().on = (enable != 0);
+  return ok();
+}
+
+int harp_ra_timing_read(double* ms, int* launches, int n_kinds) {
+  if (!ms || !launches || n_kinds < 1) return fail(HARP_RA_EINVAL, "timing_read needs output arrays");
+  for (int i = 0; i < n_kinds; ++i) {
+    ms[i] = 0.0;
+    launches[i] = 0;
+  }
+  Timing& t = timing();
+  int rc = HARP_RA_OK;
+  for (auto& r : t.recs) {
+    float e = 0.f;
+    if (hipEventElapsedTime(&e, r.a, r.b) != hipSuccess) rc = HARP_RA_ELAUNCH;
+    if (r.kind < n_kinds) {
+      ms[r.kind] += e;
+      launches[r.kind] += 1;
+    }
+    t.pool.push_back(r.a);
+    t.pool.push_back(r.b);
+  }
+  t.recs.clear();
+  if (rc) return fail(rc, "hipEventElapsedTime failed (were the streams synchronised?)");
+  return ok();
+}
+
+size_t harp_ra_forward_workspace_bytes(int batch, int h_num, int t_num, int h_len, int sp_size, int kv_chunk_len,
+                                       const int32_t* kv_valid_lens) {
+  Geometry g;
+  if (check_dims(batch, h_num, t_num, h_len) != HARP_RA_OK) return SIZE_MAX;
+  if (make_geometry(sp_size, kv_chunk_len, kv_valid_lens, &g) != HARP_RA_OK) return SIZE_MAX;
+  return fwd_ws(batch, h_num, t_num, h_len, g);
+}
+
+size_t harp_ra_backward_workspace_bytes(int batch, int h_num, int t_num, int h_len, int sp_size, int kv_chunk_len,
+                                        const int32_t* kv_valid_lens) {
+  Geometry g;
+  if (check_dims(batch, h_num, t_num, h_len) != HARP_RA_OK) return SIZE_MAX;
+  if (make_geometry(sp_size, kv_chunk_len, kv_valid_lens, &g) != HARP_RA_OK) return SIZE_MAX;
+  return bwd_ws(batch, h_num, t_num, h_len, g);
+}
+
+int harp_ra_forward(const void* q, const int64_t* q_strides, const void* const* k_chunks,
+                    const void* const* v_chunks, const int64_t* kv_strides, int kv_chunk_len,
+                    const int32_t* kv_valid_lens, float* out, const int64_t* out_strides, void* m_i, int m_i_dtype,
+                    float* l_i, int batch, int h_num, int t_num, int h_len, int sp_size, int ring_rank, float scale,
+                    void* workspace, size_t workspace_bytes, void* stream) {
+  return forward_impl(q, q_strides, k_chunks, v_chunks, kv_strides, kv_chunk_len, kv_valid_lens, out, out_strides, nullptr,
+                      nullptr, m_i, m_i_dtype, l_i, batch, h_num, t_num, h_len, sp_size, ring_rank, scale, workspace,
+                      workspace_bytes, stream);
+}
+
+int harp_ra_forward_rounded(const void* q, const int64_t* q_strides, const void* const* k_chunks,
+                            const void* const* v_chunks, const int64_t* kv_strides, int kv_chunk_len,
+                            const int32_t* kv_valid_lens, void* out_rounded, const int64_t* rounded_strides,
+                            float* out, const int64_t* out_strides, void* m_i, int m_i_dtype, float* l_i, int batch,
+                            int h_num, int t_num, int h_len, int sp_size, int ring_rank, float scale,
+                            void* workspace, size_t workspace_bytes, void* stream) {
+  if (!out_rounded) return fail(HARP_RA_EINVAL, "out_rounded is NULL");
+  return forward_impl(q, q_strides, k_chunks, v_chunks, kv_strides, kv_chunk_len, kv_valid_lens, out, out_strides,
+                      out_rounded, rounded_strides, m_i, m_i_dtype, l_i, batch, h_num, t_num, h_len, sp_size, ring_rank,
+                      scale, workspace, workspace_bytes, stream);
+}
+
+int harp_ra_delta(const void* grad_out, const int64_t* do_strides, const float* out, const int64_t* out_strides,
+                  float* delta, int batch, int h_num, int t_num, int h_len, void* stream) {
+  int rc;
+  if ((rc = check_dims(batch, h_num, t_num, h_len))) return rc;
+  if ((rc = check_bf16_view(grad_out, do_strides, h_len, "grad_out"))) return rc;
+  if ((rc = check_plain_view(out, out_strides, "out"))) return rc;
+  if (!delta) return fail(HARP_RA_EINVAL, "delta is NULL");
+  DeltaParams p;
+  p.dout = static_cast<const bf16*>(grad_out);
+  p.sdb = do_strides[0];
+  p.sdh = do_strides[1];
+  p.sdt = do_strides[2];
+  p.out = out;
+  p.sob = out_strides[0];
+  p.soh = out_strides[1];
+  p.sot = out_strides[2];
+  p.delta = delta;
+  p.B = batch;
+  p.H = h_num;
+  p.T = t_num;
+  p.D = h_len;
+  {
+    TimedLaunch tl(HARP_RA_KERNEL_DELTA, static_cast<hipStream_t>(stream));
+    if ((rc = launched(launch_delta(p, static_cast<hipStream_t>(stream)), "delta"))) return rc;
+  }
+  return ok();
+}
+
+int harp_ra_backward(const void* q, const int64_t* q_strides, void* grad_q, const int64_t* dq_strides, int dq_dtype,
+                     const void* const* k_chunks, const void* const* v_chunks, const int64_t* kv_strides,
+                     void* const* dk_chunks, void* const* dv_chunks, const int64_t* dkv_strides, int dkv_dtype,
+                     int kv_chunk_len, const int32_t* kv_valid_lens, const void* grad_out, const int64_t* do_strides,
+                     const void* m_i, int m_i_dtype, const float* l_i, const float* delta, int batch, int h_num,
+                     int t_num, int h_len, int sp_size, int ring_rank, float scale, void* workspace,
+                     size_t workspace_bytes, void* stream) {
+  if (!delta) return fail(HARP_RA_EINVAL, "m_i / l_i / delta are NULL");
+  return backward_impl(q, q_strides, grad_q, dq_strides, dq_dtype, k_chunks, v_chunks, kv_strides, dk_chunks, dv_chunks,
+                       dkv_strides, dkv_dtype, kv_chunk_len, kv_valid_lens, grad_out, do_strides, m_i, m_i_dtype, l_i,
+                       delta, nullptr, nullptr, batch, h_num, t_num, h_len, sp_size, ring_rank, scale, workspace,
+                       workspace_bytes, stream);
+}
+
+int harp_ra_backward_from_out(const void* q, const int64_t* q_strides, void* grad_q, const int64_t* dq_strides,
+                              int dq_dtype, const void* const* k_chunks, const void* const* v_chunks,
+                              const int64_t* kv_strides, void* const* dk_chunks, void* const* dv_chunks,
+                              const int64_t* dkv_strides, int dkv_dtype, int kv_chunk_len,
+                              const int32_t* kv_valid_lens, const void* grad_out, const int64_t* do_strides,
+                              const void* m_i, int m_i_dtype, const float* l_i, const float* out,
+                              const int64_t* out_strides, int batch, int h_num, int t_num, int h_len, int sp_size,
+                              int ring_rank, float scale, void* workspace, size_t workspace_bytes, void* stream) {
+  return backward_impl(q, q_strides, grad_q, dq_strides, dq_dtype, k_chunks, v_chunks, kv_strides, dk_chunks, dv_chunks,
+                       dkv_strides, dkv_dtype, kv_chunk_len, kv_valid_lens, grad_out, do_strides, m_i, m_i_dtype, l_i,
+                       nullptr, out, out_strides, batch, h_num, t_num, h_len, sp_size, ring_rank, scale, workspace,
+                       workspace_bytes, stream);
 }
 
 }  // extern "C"

@@ -12,8 +12,10 @@ struct FwdParams {
   const bf16* q;
   int64_t sqb, sqh, sqt;
   int64_t skb, skh, skt;  // strides shared by every K/V chunk
-  float* out;
+  float* out;             // fp32 O (NULL: not stored)
   int64_t sob, soh, sot;
+  bf16* outb;             // O rounded to bf16 to nearest (NULL: not stored); rows 8-byte aligned
+  int64_t sbb, sbh, sbt;
   void* m;                // [B,H,T] contiguous, fp32 or bf16
   int m_bf16;
   float* l;               // [B,H,T] contiguous
@@ -33,8 +35,10 @@ struct FwdMergeParams {
   const float* part_m;
   const float* part_l;
   int n_split;
-  float* out;
+  float* out;  // as FwdParams: out and outb may be NULL
   int64_t sob, soh, sot;
+  bf16* outb;
+  int64_t sbb, sbh, sbt;
   void* m;
   int m_bf16;
   float* l;
@@ -74,7 +78,9 @@ struct BwdParams {
   const void* m;
   int m_bf16;
   const float* l;
-  const float* delta;
+  const float* delta;          // [B,H,T] contiguous; NULL: the dQ kernel forms it from dO and out
+  const float* out;            // the forward's fp32 O (read only when delta is NULL)
+  int64_t sob, soh, sot;
   float* stats;             // workspace [2][B*H*T]: -(m + ln l) / scale, -D (written by the dQ kernel)
   int n_split;              // KV splits of the dQ kernel (grid dimension y); > 1: dq is per-split partials
   int64_t split_dq;         // elements between the splits' dQ buffers

@@ -594,7 +594,8 @@ __global__ __launch_bounds__(64 * kFwdWaves, 1) void fwd_kernel(FwdParams p) {
         *(f32x4*)(st + E::stage_write_tail(u, lane_e)) = ot[u] * __shfl(inv, 16 * u + (lane_e & 15));
     }
     __syncthreads();
-    float* const ob = p.out + sp.index * p.split_o + (int64_t)b * p.sob + (int64_t)h * p.soh;
+    const int64_t bh = sp.index * p.split_o + (int64_t)b * p.sob + (int64_t)h * p.soh;
+    const int64_t bhb = (int64_t)b * p.sbb + (int64_t)h * p.sbh;
     const int q0 = qt * kFwdRows + wave * 32;
 #pragma unroll
     for (int it0 = 0; it0 < E::kIters; it0 += 4) {
@@ -607,22 +608,28 @@ __global__ __launch_bounds__(64 * kFwdWaves, 1) void fwd_kernel(FwdParams p) {
         if (it0 + j >= E::kIters) break;  // a last group of fewer than four (16-wide d tail)
         const int qi = q0 + E::read_row(it0 + j, lane_e), ch = E::read_chunk(it0 + j, lane_e);
         if (qi >= p.T || 4 * ch >= p.D) continue;
-        float* const o4 = ob + (int64_t)qi * p.sot + 4 * ch;
-        o4[0] = x[j].x;
-        o4[1] = x[j].y;
-        o4[2] = x[j].z;
-        o4[3] = x[j].w;
+        if (p.out) {
+          float* const o4 = p.out + bh + (int64_t)qi * p.sot + 4 * ch;
+          o4[0] = x[j].x;
+          o4[1] = x[j].y;
+          o4[2] = x[j].z;
+          o4[3] = x[j].w;
+        }
+        if (p.outb) *(bf16x4*)(p.outb + bhb + (int64_t)qi * p.sbt + 4 * ch) = __builtin_convertvector(x[j], bf16x4);
       }
     }
   } else if (qi_e < p.T) {
     static_assert(!kTail, "the tail variant always fits the staged epilogue");
-    float* orow = p.out + sp.index * p.split_o + (int64_t)b * p.sob + (int64_t)h * p.soh + (int64_t)qi_e * p.sot;
+    const int64_t row = sp.index * p.split_o + (int64_t)b * p.sob + (int64_t)h * p.soh + (int64_t)qi_e * p.sot;
+    const int64_t rowb = (int64_t)b * p.sbb + (int64_t)h * p.sbh + (int64_t)qi_e * p.sbt;
 #pragma unroll
     for (int db = 0; db < DBF; ++db)
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         const int d = db * 32 + c_row(r, g_e);
-        if (d < p.D) orow[d] = o[db][r] * inv;
+        if (d >= p.D) continue;
+        if (p.out) p.out[row + d] = o[db][r] * inv;
+        if (p.outb) p.outb[rowb + d] = (bf16)(o[db][r] * inv);
       }
   }
   if (qi_e < p.T && g_e == 0) {
@@ -742,7 +749,28 @@ __global__ __launch_bounds__(64 * kDqWaves, 1) void dq_kernel(BwdParams p) {
   // the row's statistics (bwd_stat_lse), written once for the dK/dV kernel;
   // LSE2 = -c * plane 0 (+inf for a row without keys); D = -plane 1
   const float st0 = q_ok ? bwd_stat_lse(p, si) : 0.f;
-  const float st1 = q_ok ? -p.delta[si] : 0.f;
+  float st1 = 0.f;
+  if (p.delta) {
+    if (q_ok) st1 = -p.delta[si];
+  } else {
+    // D = rowsum(dO O) here, from the dO fragments the lane holds anyway (its
+    // two lane halves each cover half of the row): no launch for it
+    float acc = 0.f;
+    const float* orow = p.out + (int64_t)b * p.sob + (int64_t)h * p.soh + (int64_t)qi * p.sot;
+#pragma unroll
+    for (int ks = 0; ks < KSTEPS; ++ks) {
+      const int d0 = ks * 16 + g * 8;
+      if (q_ok && d0 < p.D) {
+        const f32x4u x = *(const f32x4u*)(orow + d0), y = *(const f32x4u*)(orow + d0 + 4);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          acc = __builtin_fmaf((float)gf[ks][j], x[j], acc);
+          acc = __builtin_fmaf((float)gf[ks][j + 4], y[j], acc);
+        }
+      }
+    }
+    st1 = -wave_half_sum(acc);
+  }
   if (q_ok && g == 0 && sp.index == 0) {
     p.stats[si] = st0;
     p.stats[nrows + si] = st1;
@@ -1441,9 +1469,19 @@ __global__ __launch_bounds__(256) void fwd_merge_kernel(FwdMergeParams p) {
   const int h = (int)(bh % p.H), b = (int)(bh / p.H);
   const float inv = (l > 0.f) ? 1.f / l : 0.f;
   if (has_d) {
-    float* orow = p.out + (int64_t)b * p.sob + (int64_t)h * p.soh + (int64_t)t * p.sot + d0;
+    if (p.out) {
+      float* orow = p.out + (int64_t)b * p.sob + (int64_t)h * p.soh + (int64_t)t * p.sot + d0;
 #pragma unroll
-    for (int j = 0; j < 8; ++j) orow[j] = acc[j] * inv;
+      for (int j = 0; j < 8; ++j) orow[j] = acc[j] * inv;
+    }
+    if (p.outb) {
+      bf16* brow = p.outb + (int64_t)b * p.sbb + (int64_t)h * p.sbh + (int64_t)t * p.sbt + d0;
+#pragma unroll
+      for (int j = 0; j < 8; j += 4) {
+        const f32x4 x = {acc[j] * inv, acc[j + 1] * inv, acc[j + 2] * inv, acc[j + 3] * inv};
+        *(bf16x4*)(brow + j) = __builtin_convertvector(x, bf16x4);
+      }
+    }
   }
   if (sub == 0) {  // statistics as the forward kernel writes them
     if (p.m_bf16) {

@@ -11,7 +11,17 @@
 //                           sp_size, scale, ring_rank=0, kv_lens=None,
 //                           kv_chunk_len=0)
 // plus ring_attention_delta(grad_out, out) -> D, the rowsum(dO*O) preprocess
-// of src/models/z_image/module/attn.py:41 as one kernel.
+// of src/models/z_image/module/attn.py:41 as one kernel, and
+//   ring_attention_attend(q, k, v, sp_size, scale, ring_rank=0, kv_lens=None,
+//                         kv_chunk_len=0, keep_for_backward=True)
+//     -> (o, out, m_i, l_i)
+//   ring_attention_grad(grad_out, q, k, v, out, m_i, l_i, sp_size, scale,
+//                       ring_rank=0, kv_lens=None, kv_chunk_len=0)
+//     -> (dq, dk, dv)
+// the bodies of CPURingAttention's forward and backward (attn.py:16-49) as one
+// call each: the outputs allocated here, O rounded to bf16 by the kernel that
+// computes it, and D formed inside the dQ kernel, so neither direction
+// launches anything but the attention kernels.
 //
 // Implementations are registered for the CUDA dispatch key (PyTorch-ROCm
 // tensors on a HIP device carry it) and call libharp_ra.so through its C ABI
@@ -228,6 +238,101 @@ std::tuple<at::Tensor, at::Tensor, at::Tensor> backward_hip(const at::Tensor& q,
   return std::make_tuple(grad_q, dK, dV);
 }
 
+// forward of CPURingAttention (attn.py:16-33): o = out rounded to bf16, with
+// q's strides as empty_like gives them; out (fp32) only when a backward follows
+std::tuple<at::Tensor, at::Tensor, at::Tensor, at::Tensor> attend_hip(const at::Tensor& q, const at::Tensor& k,
+                                                                      const at::Tensor& v, int64_t sp_size,
+                                                                      double scale, int64_t ring_rank,
+                                                                      at::OptionalIntArrayRef kv_lens,
+                                                                      int64_t kv_chunk_len, bool keep) {
+  check_bhtd(q, "q");
+  check_bhtd(k, "k");
+  check_bhtd(v, "v");
+  check_device(k, q, "tensor");
+  check_device(v, q, "tensor");
+  TORCH_CHECK(q.scalar_type() == at::kBFloat16 && k.scalar_type() == at::kBFloat16 &&
+                  v.scalar_type() == at::kBFloat16,
+              "q, k, v must be bfloat16");
+  Chunks ch = split_chunks("ring_attention_forward", q, k, v, sp_size, kv_lens, kv_chunk_len);
+  const c10::DeviceGuard guard(q.device());
+  const int B = q.size(0), H = q.size(1), T = q.size(2), D = q.size(3);
+  const int32_t* lens = ch.lens.empty() ? nullptr : ch.lens.data();
+  const size_t ws_bytes = harp_ra_forward_workspace_bytes(B, H, T, D, sp_size, ch.chunk_len, lens);
+  check_status(ws_bytes != SIZE_MAX ? HARP_RA_OK : HARP_RA_EINVAL, "ring_attention_forward");
+  at::Tensor o = at::empty_like(q);
+  at::Tensor out = keep ? at::empty_like(q, q.options().dtype(at::kFloat)) : at::empty({0}, q.options().dtype(at::kFloat));
+  at::Tensor m_i = at::empty({B, H, T, 1}, q.options());
+  at::Tensor l_i = at::empty({B, H, T, 1}, q.options().dtype(at::kFloat));
+  at::Tensor ws = workspace(ws_bytes, q);
+  const auto qs = strides4(q), ks = strides4(k), bs = strides4(o);
+  std::array<int64_t, 4> os{};
+  if (keep) os = strides4(out);
+  hipStream_t stream = c10::hip::getCurrentHIPStream(q.get_device()).stream();
+  const int rc = harp_ra_forward_rounded(
+      q.data_ptr(), qs.data(), ch.k.data(), ch.v.data(), ks.data(), ch.chunk_len, lens, o.data_ptr(), bs.data(),
+      keep ? out.data_ptr<float>() : nullptr, os.data(), m_i.data_ptr(), HARP_RA_BF16, l_i.data_ptr<float>(), B, H, T,
+      D, static_cast<int>(sp_size), static_cast<int>(ring_rank), static_cast<float>(scale), ws_ptr(ws), ws_bytes,
+      stream);
+  check_status(rc, "ring_attention_forward");
+  return std::make_tuple(o, out, m_i, l_i);
+}
+
+// grad_out as the kernels read it in place (bf16, unit D stride, other strides
+// multiples of 8 elements, 16-byte aligned), else a copy
+at::Tensor kernel_view(const at::Tensor& t) {
+  at::Tensor x = t.to(at::kBFloat16);
+  bool ok = x.stride(3) == 1 && reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 == 0;
+  for (int i = 0; i < 3; ++i) ok = ok && x.stride(i) % 8 == 0 && x.stride(i) >= 0;
+  return ok ? x : x.contiguous();
+}
+
+// backward of CPURingAttention (attn.py:35-49); the gradients take the
+// strides of q, k and v as empty_like gives them
+std::tuple<at::Tensor, at::Tensor, at::Tensor> grad_hip(const at::Tensor& grad_out, const at::Tensor& q,
+                                                        const at::Tensor& k, const at::Tensor& v,
+                                                        const at::Tensor& out, const at::Tensor& m_i,
+                                                        const at::Tensor& l_i, int64_t sp_size, double scale,
+                                                        int64_t ring_rank, at::OptionalIntArrayRef kv_lens,
+                                                        int64_t kv_chunk_len) {
+  for (const at::Tensor* t : {&q, &k, &v, &grad_out}) check_bhtd(*t, "gradient operand");
+  check_bhtd(out, "out");
+  for (const at::Tensor* t : {&k, &v, &grad_out, &out, &m_i, &l_i}) check_device(*t, q, "tensor");
+  TORCH_CHECK(q.scalar_type() == at::kBFloat16 && k.scalar_type() == at::kBFloat16 &&
+                  v.scalar_type() == at::kBFloat16,
+              "q, k, v, grad_out must be bfloat16");
+  TORCH_CHECK(grad_out.sizes() == q.sizes(), "grad_out must have q's shape");
+  TORCH_CHECK(out.sizes() == q.sizes() && out.scalar_type() == at::kFloat, "out must be float32 with q's shape");
+  check_stats(m_i, q, "m_i");
+  check_stats(l_i, q, "l_i");
+  TORCH_CHECK(l_i.scalar_type() == at::kFloat, "l_i and D must be float32");
+  const int m_code = dtype_code(m_i, "m_i");
+  const c10::DeviceGuard guard(q.device());
+  const at::Tensor g = kernel_view(grad_out);
+  at::Tensor dq = at::empty_like(q), dk = at::empty_like(k), dv = at::empty_like(v);
+  TORCH_CHECK(dk.strides() == dv.strides(), "dK and dV must have the same strides");
+  Chunks ch = split_chunks("ring_attention_backward", q, k, v, sp_size, kv_lens, kv_chunk_len);
+  const int64_t dstep = ch.chunk_len * dk.stride(2) * dk.element_size();
+  for (int64_t i = 0; i < sp_size; ++i) {
+    ch.dk.push_back(static_cast<char*>(dk.data_ptr()) + i * dstep);
+    ch.dv.push_back(static_cast<char*>(dv.data_ptr()) + i * dstep);
+  }
+  const int B = q.size(0), H = q.size(1), T = q.size(2), Dh = q.size(3);
+  const int32_t* lens = ch.lens.empty() ? nullptr : ch.lens.data();
+  const size_t ws_bytes = harp_ra_backward_workspace_bytes(B, H, T, Dh, sp_size, ch.chunk_len, lens);
+  check_status(ws_bytes != SIZE_MAX ? HARP_RA_OK : HARP_RA_EINVAL, "ring_attention_backward");
+  at::Tensor ws = workspace(ws_bytes, q);
+  const auto qs = strides4(q), dqs = strides4(dq), ks = strides4(k), dks = strides4(dk), gs = strides4(g),
+             os = strides4(out);
+  hipStream_t stream = c10::hip::getCurrentHIPStream(q.get_device()).stream();
+  const int rc = harp_ra_backward_from_out(
+      q.data_ptr(), qs.data(), dq.data_ptr(), dqs.data(), HARP_RA_BF16, ch.k.data(), ch.v.data(), ks.data(),
+      ch.dk.data(), ch.dv.data(), dks.data(), HARP_RA_BF16, ch.chunk_len, lens, g.data_ptr(), gs.data(),
+      m_i.data_ptr(), m_code, l_i.data_ptr<float>(), out.data_ptr<float>(), os.data(), B, H, T, Dh,
+      static_cast<int>(sp_size), static_cast<int>(ring_rank), static_cast<float>(scale), ws_ptr(ws), ws_bytes, stream);
+  check_status(rc, "ring_attention_backward");
+  return std::make_tuple(dq, dk, dv);
+}
+
 at::Tensor delta_hip(const at::Tensor& grad_out, const at::Tensor& out) {
   check_bhtd(grad_out, "grad_out");
   check_bhtd(out, "out");
@@ -273,6 +378,26 @@ std::tuple<at::Tensor, at::Tensor, at::Tensor> backward_cpu(const at::Tensor& q,
   (void)split_chunks("ring_attention_backward", q, k, v, sp_size, kv_lens, kv_chunk_len);
   no_cpu_path("ring_attention_backward");
 }
+std::tuple<at::Tensor, at::Tensor, at::Tensor, at::Tensor> attend_cpu(const at::Tensor& q, const at::Tensor& k,
+                                                                      const at::Tensor& v, int64_t sp_size, double,
+                                                                      int64_t, at::OptionalIntArrayRef kv_lens,
+                                                                      int64_t kv_chunk_len, bool) {
+  check_bhtd(q, "q");
+  check_bhtd(k, "k");
+  check_bhtd(v, "v");
+  (void)split_chunks("ring_attention_forward", q, k, v, sp_size, kv_lens, kv_chunk_len);
+  no_cpu_path("ring_attention_forward");
+}
+std::tuple<at::Tensor, at::Tensor, at::Tensor> grad_cpu(const at::Tensor&, const at::Tensor& q, const at::Tensor& k,
+                                                        const at::Tensor& v, const at::Tensor&, const at::Tensor&,
+                                                        const at::Tensor&, int64_t sp_size, double, int64_t,
+                                                        at::OptionalIntArrayRef kv_lens, int64_t kv_chunk_len) {
+  check_bhtd(q, "q");
+  check_bhtd(k, "k");
+  check_bhtd(v, "v");
+  (void)split_chunks("ring_attention_backward", q, k, v, sp_size, kv_lens, kv_chunk_len);
+  no_cpu_path("ring_attention_backward");
+}
 at::Tensor delta_cpu(const at::Tensor&, const at::Tensor&) { no_cpu_path("ring_attention_delta"); }
 
 }  // namespace
@@ -287,16 +412,26 @@ TORCH_LIBRARY(ring_attention_ops, m) {
       "Tensor grad_out, Tensor m_i, Tensor l_i, Tensor D, int sp_size, float scale, int ring_rank=0, "
       "int[]? kv_lens=None, int kv_chunk_len=0) -> (Tensor(a!), Tensor(b!), Tensor(c!))");
   m.def("ring_attention_delta(Tensor grad_out, Tensor out) -> Tensor");
+  m.def(
+      "ring_attention_attend(Tensor q, Tensor k, Tensor v, int sp_size, float scale, int ring_rank=0, "
+      "int[]? kv_lens=None, int kv_chunk_len=0, bool keep_for_backward=True) -> (Tensor, Tensor, Tensor, Tensor)");
+  m.def(
+      "ring_attention_grad(Tensor grad_out, Tensor q, Tensor k, Tensor v, Tensor out, Tensor m_i, Tensor l_i, "
+      "int sp_size, float scale, int ring_rank=0, int[]? kv_lens=None, int kv_chunk_len=0) -> (Tensor, Tensor, Tensor)");
 }
 
 TORCH_LIBRARY_IMPL(ring_attention_ops, CUDA, m) {
   m.impl("ring_attention_forward", &forward_hip);
   m.impl("ring_attention_backward", &backward_hip);
   m.impl("ring_attention_delta", &delta_hip);
+  m.impl("ring_attention_attend", &attend_hip);
+  m.impl("ring_attention_grad", &grad_hip);
 }
 
 TORCH_LIBRARY_IMPL(ring_attention_ops, CPU, m) {
   m.impl("ring_attention_forward", &forward_cpu);
   m.impl("ring_attention_backward", &backward_cpu);
   m.impl("ring_attention_delta", &delta_cpu);
+  m.impl("ring_attention_attend", &attend_cpu);
+  m.impl("ring_attention_grad", &grad_cpu);
 }

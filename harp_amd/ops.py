@@ -2,10 +2,11 @@
 
 * :class:`RingAttention` mirrors ``CPURingAttention``
   (src/models/z_image/module/attn.py:15-49): same arguments, same caller-
-  allocated ``out`` (fp32, q's token-major strides), bf16 ``m_i`` and fp32
-  ``l_i``, same saved tensors, same ``D = rowsum(dO * O)`` preprocess (here one
-  kernel, ``ring_attention_delta``), same op calls by name through
-  ``torch.ops.ring_attention_ops``.
+  ``out`` (fp32, q's token-major strides), bf16 ``m_i`` and fp32 ``l_i``, same
+  saved tensors, same ``D = rowsum(dO * O)``.  Each direction is one operator
+  call (``ring_attention_attend``, ``ring_attention_grad`` of
+  ``torch.ops.ring_attention_ops``): the allocations are native, the kernels
+  store the rounded output themselves and form D where it is used.
 * :func:`abi_forward` / :func:`abi_backward` / :func:`abi_delta` call
   libharp_ra.so's C ABI directly (ctypes), with per-chunk pointers, so the KV
   chunks of the ring need not be contiguous.
@@ -45,42 +46,26 @@ class RingAttention(torch.autograd.Function):
         ctx.chunk_len = local_k.size(2) // sp_size
         scale = 1.0 / math.sqrt(local_q.size(-1))  # attn.py:20
         ctx.scale = scale
-        mm_type = local_q.dtype
-        B, H, T, _ = local_q.shape
-        # attn.py:24-27 allocates out with zeros_like (token-major strides); every
-        # element is written by the kernel, so empty_like keeps the layout without a fill
-        out = torch.empty_like(local_q, dtype=torch.float32)
-        m_i = torch.full((B, H, T, 1), float("-inf"), device=local_q.device, dtype=torch.bfloat16)
-        l_i = torch.empty((B, H, T, 1), device=local_q.device, dtype=torch.float32)
-        _ops().ring_attention_forward(local_q, local_k, local_v, out, m_i, l_i, sp_size, scale, ring_rank, kv_lens,
-                                      ctx.chunk_len)
-        ctx.save_for_backward(local_q, local_k, local_v, out, m_i, l_i)
-        return out.to(mm_type)
+        # attn.py:24-32: out, m_i and l_i are allocated, filled and out is cast
+        # to q's dtype; the operator allocates them in the same layouts and its
+        # kernel stores both forms of out.  Without a gradient to take, the
+        # fp32 one is neither stored nor kept.
+        keep = any(ctx.needs_input_grad)
+        o, out, m_i, l_i = _ops().ring_attention_attend(local_q, local_k, local_v, sp_size, scale, ring_rank, kv_lens,
+                                                        ctx.chunk_len, keep)
+        if keep:
+            ctx.save_for_backward(local_q, local_k, local_v, out, m_i, l_i)
+        return o
 
     @staticmethod
     def backward(ctx, grad_out):
         local_q, local_k, local_v, out, m_i, l_i = ctx.saved_tensors
-        grad_out = _kernel_view(grad_out.to(torch.bfloat16))
-        D = _ops().ring_attention_delta(grad_out, out)  # attn.py:41
-        grad_q = torch.empty_like(local_q, dtype=torch.bfloat16)
-        grad_k = torch.empty_like(local_k, dtype=torch.bfloat16)
-        grad_v = torch.empty_like(local_v, dtype=torch.bfloat16)
-        _ops().ring_attention_backward(
-            local_q, grad_q, local_k, grad_k, local_v, grad_v, grad_out, m_i, l_i, D,
+        # attn.py:41-47: D, the gradients' allocation and the backward in one call
+        grad_q, grad_k, grad_v = _ops().ring_attention_grad(
+            grad_out, local_q, local_k, local_v, out, m_i, l_i,
             ctx.sp_size, ctx.scale, ctx.ring_rank, ctx.kv_lens, ctx.chunk_len,
         )
         return grad_q, grad_k, grad_v, None, None, None
-
-
-def _kernel_view(t: torch.Tensor) -> torch.Tensor:
-    """Return ``t`` if the kernels can read it in place (unit D stride, other
-    strides multiples of 8 elements, 16-byte aligned), else a contiguous copy."""
-    ok = (
-        t.stride(3) == 1
-        and all(s % 8 == 0 and s >= 0 for s in t.stride()[:3])
-        and t.data_ptr() % 16 == 0
-    )
-    return t if ok else t.contiguous()
 
 
 def ring_attention(q, k, v, sp_size: int, ring_rank: int = 0, kv_lens: Optional[Sequence[int]] = None):

@@ -76,6 +76,26 @@ HARP_RA_API int harp_ra_forward(const void* q, const int64_t* q_strides,
                     void* workspace, size_t workspace_bytes, void* stream);
 
 /*
+ * harp_ra_forward whose kernels also (or, with out NULL, only) store O rounded
+ * to bf16 to nearest: what a caller that casts out afterwards (as
+ * CPURingAttention.forward does, src/models/z_image/module/attn.py:32) would
+ * read 4 bytes and write 2 per element for.  out_rounded is a [B,H,T,D] view
+ * as out, its pointer 8-byte aligned and its strides (of dims longer than 1)
+ * multiples of 4 elements; out may be NULL (its strides are then ignored) when
+ * no backward follows.  Everything else as harp_ra_forward.
+ */
+HARP_RA_API int harp_ra_forward_rounded(const void* q, const int64_t* q_strides,
+                    const void* const* k_chunks, const void* const* v_chunks,
+                    const int64_t* kv_strides, int kv_chunk_len,
+                    const int32_t* kv_valid_lens,
+                    void* out_rounded, const int64_t* rounded_strides,
+                    float* out, const int64_t* out_strides,
+                    void* m_i, int m_i_dtype, float* l_i,
+                    int batch, int h_num, int t_num, int h_len,
+                    int sp_size, int ring_rank, float scale,
+                    void* workspace, size_t workspace_bytes, void* stream);
+
+/*
  * Backward of one rank's share: dQ for the local rows and Q_local's
  * contribution to dK/dV of every chunk (pad keys receive 0), accumulated in
  * fp32 and written once as fp32 or bf16 (dq_dtype / dkv_dtype).  P is
@@ -105,6 +125,26 @@ HARP_RA_API int harp_ra_backward(const void* q, const int64_t* q_strides,
                      const void* grad_out, const int64_t* do_strides,
                      const void* m_i, int m_i_dtype, const float* l_i,
                      const float* delta,
+                     int batch, int h_num, int t_num, int h_len,
+                     int sp_size, int ring_rank, float scale,
+                     void* workspace, size_t workspace_bytes, void* stream);
+
+/*
+ * harp_ra_backward without a delta argument: the dQ kernel forms
+ * rowsum(dO * O) in fp32 from grad_out and `out`, the fp32 output of the
+ * forward (a view with unit D stride, as harp_ra_delta takes it), so the
+ * caller launches no harp_ra_delta.  Everything else as harp_ra_backward.
+ */
+HARP_RA_API int harp_ra_backward_from_out(const void* q, const int64_t* q_strides,
+                     void* grad_q, const int64_t* dq_strides, int dq_dtype,
+                     const void* const* k_chunks, const void* const* v_chunks,
+                     const int64_t* kv_strides,
+                     void* const* dk_chunks, void* const* dv_chunks,
+                     const int64_t* dkv_strides, int dkv_dtype,
+                     int kv_chunk_len, const int32_t* kv_valid_lens,
+                     const void* grad_out, const int64_t* do_strides,
+                     const void* m_i, int m_i_dtype, const float* l_i,
+                     const float* out, const int64_t* out_strides,
                      int batch, int h_num, int t_num, int h_len,
                      int sp_size, int ring_rank, float scale,
                      void* workspace, size_t workspace_bytes, void* stream);

@@ -267,7 +267,7 @@ int backward(int mode, const void* dy, const int64_t* dys, const void* x, const 
   p.wpart = static_cast<float*>(ws);
   if ((rc = launched(launch_qk_backward(p, mode, st), "QK backward"))) return rc;
   if ((mode & 1) && gw) {
-    if ((rc = launched(launch_wgrad_reduce(p.wpart, bwd_blocks(sh), D, gw, gwdt == HARP_QK_F32, st),
+    if ((rc = launched(launch_wgrad_reduce(p.wpart, bwd_launch_blocks(sh), D, gw, gwdt == HARP_QK_F32, st),
                        "weight-gradient reduction")))
       return rc;
   }

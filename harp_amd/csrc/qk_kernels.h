@@ -28,6 +28,16 @@ struct QkFwdParams {
   int64_t f_stride_b, f_stride_s;
 };
 
+struct RopeParams {
+  QkShape sh;
+  const uint16_t* x;
+  Strides4 sx;
+  uint16_t* out;
+  Strides4 so;
+  const float* freqs;
+  int64_t f_stride_b, f_stride_s;
+};
+
 struct QkBwdParams {
   QkShape sh;
   const uint16_t* dy;  // gradient of the op's output, bf16
@@ -41,17 +51,21 @@ struct QkBwdParams {
   const float* rms;    // saved by the forward
   const float* freqs;
   int64_t f_stride_b, f_stride_s;
-  float* wpart;        // [blocks][D] fp32 weight-gradient partials, then the
-                       // reduction's group sums (workspace, bwd_workspace_floats)
+  float* wpart;        // [blocks][D] fp32 weight-gradient partials (workspace)
 };
 
-// Blocks of the backward kernel (each a contiguous range of rows); bounds the
-// weight-gradient workspace (one partial row of D floats per block).
+// The weight-gradient workspace (harp_qk_backward_workspace_bytes): one
+// partial row of D floats for each of up to kQkBwdMaxBlocks 16-row blocks,
+// and one row more per kWgGroupRows of them.
 constexpr int kQkBwdMaxBlocks = 2048;
 int bwd_blocks(const QkShape& sh);
-// Partial rows per group of the first level of the weight-gradient reduction;
-// the workspace holds the partials and then one row per group.
 constexpr int kWgGroupRows = 64;
+// Blocks the backward kernel is launched with (each a contiguous range of
+// rows, one partial row), never more than bwd_blocks.
+// (1024: four 4-wave blocks per CU; the forward's registers fit eight)
+constexpr int kQkBwdMaxLaunch = 1024;
+constexpr int kQkFwdMaxLaunch = 2048;
+int bwd_launch_blocks(const QkShape& sh);
 inline size_t bwd_workspace_floats(const QkShape& sh) {
   const size_t nblk = (size_t)bwd_blocks(sh);
   return (nblk + (nblk + kWgGroupRows - 1) / kWgGroupRows) * (size_t)sh.D;

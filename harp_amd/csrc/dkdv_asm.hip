@@ -165,14 +165,15 @@ __global__ __launch_bounds__(64 * kAsmWaves, 1) void dkdv_asm_kernel(BwdParams p
     for (int i = 0; i < 32; ++i) misc[i] = mv[i];
   }
 
-  const int nb = any ? (p.T + 31) >> 5 : 0;
-  const bf16* qb = p.q + (int64_t)b * p.sqb + (int64_t)h * p.sqh;
-  const bf16* gb = p.dout + (int64_t)b * p.sdb + (int64_t)h * p.sdh;
-  const int64_t sbase = ((int64_t)b * p.H + h) * p.T;
+  const QSplit qs = q_split(p);
+  const int nb = any ? (qs.rows + 31) >> 5 : 0;
+  const bf16* qb = p.q + (int64_t)b * p.sqb + (int64_t)h * p.sqh + qs.begin * p.sqt;
+  const bf16* gb = p.dout + (int64_t)b * p.sdb + (int64_t)h * p.sdh + qs.begin * p.sdt;
+  const int64_t sbase = ((int64_t)b * p.H + h) * p.T + qs.begin;
   const int64_t nrows = (int64_t)p.B * p.H * p.T;
   const uint64_t qp = (uint64_t)(uintptr_t)qb, gp = (uint64_t)(uintptr_t)gb;
   const uint64_t sp0 = (uint64_t)(uintptr_t)(p.stats + sbase), sp1 = (uint64_t)(uintptr_t)(p.stats + nrows + sbase);
-  const uint32_t qnr = (uint32_t)(p.T * qrow), gnr = (uint32_t)(p.T * grow), snr = (uint32_t)(p.T * 4);
+  const uint32_t qnr = (uint32_t)(qs.rows * qrow), gnr = (uint32_t)(qs.rows * grow), snr = (uint32_t)(qs.rows * 4);
   const uint32_t qstep = (uint32_t)(32 * qrow), gstep = (uint32_t)(32 * grow);
   const uint32_t dbase = lds0 + (uint32_t)wave * 2048u;
   const uint32_t stb = lds0 + kStatsOff + (uint32_t)wave * kStatsPerWave;
@@ -251,17 +252,13 @@ __global__ __launch_bounds__(64 * kAsmWaves, 1) void dkdv_asm_kernel(BwdParams p
         const int t = kg * 2 + (db >> 1), idx = (db & 1) * 16 + r;
         const v32i& dkt = t == 0 ? o0 : (t == 1 ? o1 : (t == 2 ? o2 : o3));
         const v32i& dvt = t == 0 ? o4 : (t == 1 ? o5 : (t == 2 ? o6 : o7));
-        const int64_t e = base + (int64_t)kk * p.sdkt + d;
+        // only fp32 outputs, the query splits' partials among them, come here
+        const int64_t e = base + (int64_t)blockIdx.y * p.split_dkv + (int64_t)kk * p.sdkt + d;
         const bool valid = kk < len;
         const float vk = valid ? __int_as_float(dkt[idx]) * p.scale : 0.f;
         const float vv = valid ? __int_as_float(dvt[idx]) : 0.f;
-        if (p.dkv_f32) {
-          ((float*)p.ct.dk[c])[e] = vk;
-          ((float*)p.ct.dv[c])[e] = vv;
-        } else {
-          p.ct.dk[c][e] = (bf16)vk;
-          p.ct.dv[c][e] = (bf16)vv;
-        }
+        ((float*)p.ct.dk[c])[e] = vk;
+        ((float*)p.ct.dv[c])[e] = vv;
       }
     }
 }
@@ -274,7 +271,7 @@ bool dkdv_asm_applies(const BwdParams& p) {
 
 hipError_t launch_dkdv_asm(const BwdParams& p, hipStream_t st) {
   const int n = p.n_key_tiles * p.H * p.B;
-  hipLaunchKernelGGL(dkdv_asm_kernel, dim3(n), dim3(64 * kAsmWaves), 0, st, p);
+  hipLaunchKernelGGL(dkdv_asm_kernel, dim3(n, p.n_split), dim3(64 * kAsmWaves), 0, st, p);
   return hipGetLastError();
 }
 

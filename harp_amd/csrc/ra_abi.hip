@@ -170,31 +170,134 @@ int device_cus() {
   return cus;
 }
 
-// KV splits of the forward and dQ kernels.  Their grids have one 8-wave
-// block (one CU) per 256-query tile and (b, h); when that leaves at least
-// half of the CUs idle, each tile's ring steps are split over up to N blocks
-// (never more splits than chunks), whose partial results are merged after.
-int kv_splits(int batch, int h_num, int t_num, const Geometry& g) {
-  const int64_t blocks = (int64_t)((t_num + kQueryBlockRows - 1) / kQueryBlockRows) * h_num * batch;
+// Splits of the attention kernels' grids.  A forward / dQ grid has one block
+// (one CU) per 256-query tile and (b, h), a dK/dV grid one per 256 keys; when
+// that leaves at least half of the CUs idle, each block's stream (its keys; its
+// queries) is split over several blocks, whose fp32 partial results a second
+// launch merges.  Whether that pays follows from what was measured on the
+// MI355X: on a busy chip a block takes 0.02-0.028 us per key of its stream in
+// the forward, 0.03-0.035 in dQ and 0.038-0.048 per query in dK/dV, at head
+// dims 64 to 128, beside a fixed 8-10 us, and a merge launch 4.5 us of the GPU
+// + the partials' bytes, written and read, at about 5 TB/s.  The rest of
+// kMergeUs is the launch's cost on the host, which bounds calls this small: 8
+// heads x 512 x 512 at head dim 64, forward + backward through autograd, took
+// 94 us whole and 105 with its three grids split in two, although their GPU
+// time fell from 48 to 45.
+constexpr double kFwdUsPerKey = 0.028, kDqUsPerKey = 0.035, kDkdvUsPerQuery = 0.045;
+constexpr double kMergeUs = 10., kMergeBytesPerUs = 5e6;
+// fewer keys or queries than this per block are all fixed cost
+constexpr int kMinStream = 256;
+constexpr int kMaxQSplits = 8;
+
+// CUs per block of a grid, when at least two (else 1: no split)
+int grid_fill(int64_t blocks) {
   const int cus = device_cus();
-  if (g.n < 2 || cus < 2 || blocks * 2 > cus) return 1;
-  const int64_t fill = cus / blocks;
-  return (int)(fill < g.n ? fill : g.n);
+  return cus >= 2 && blocks * 2 <= cus ? (int)(cus / blocks) : 1;
+}
+
+// Microseconds of a stream of `len` (in units of `us`) run in `n` splits of at
+// most `part`, with `bytes` of partial results written and read per split.
+double split_cost(double us, int64_t part, int n, double bytes) {
+  return us * (double)part + (n > 1 ? kMergeUs + n * bytes / kMergeBytesPerUs : 0.);
+}
+
+// KV splits of the forward and dQ kernels: the ring steps over up to N blocks
+// or, where the CUs hold every step's block twice or more, also each step's
+// keys, in `pieces` runs of `piece` keys (a multiple of 128, the longest key
+// tile).  30 heads x 1024 queries x 1024 keys of one chunk stay whole (two
+// pieces: 33.2 us against 32.0); 8 heads x 1500 x 1500 take four pieces, the
+// forward 38.8 -> 32.8 us at head dim 128 and 30 -> 22 at 64; 8 heads x 4096 x
+// 4096 two, 95 -> 80.
+struct KvPlan {
+  int n_split;
+  int pieces;  // per chunk
+  int piece;   // keys per piece (pieces > 1)
+};
+KvPlan kv_plan(double us_per_key, int batch, int h_num, int t_num, int h_len, const Geometry& g) {
+  KvPlan best{1, 1, 0};
+  const int fill = grid_fill((int64_t)((t_num + kQueryBlockRows - 1) / kQueryBlockRows) * h_num * batch);
+  int longest = 0;
+  int64_t keys = 0;
+  for (int c = 0; c < g.n; ++c) {
+    longest = g.len[c] > longest ? g.len[c] : longest;
+    keys += g.len[c];
+  }
+  const double bytes = 8. * batch * h_num * t_num * h_len;  // one fp32 partial, written and read
+  double cost = split_cost(us_per_key, keys, 1, bytes);
+  for (int n = 2; n <= fill && n <= g.n; ++n) {  // whole ring steps
+    const double c = split_cost(us_per_key, (int64_t)((g.n + n - 1) / n) * longest, n, bytes);
+    if (c < cost) {
+      cost = c;
+      best = KvPlan{n, 1, 0};
+    }
+  }
+  for (int m = 2; m <= fill / g.n && m <= kMaxChunks / g.n && m <= longest / kMinStream; ++m) {
+    const int piece = ((longest + m - 1) / m + 127) / 128 * 128, pieces = (longest + piece - 1) / piece;
+    const double c = split_cost(us_per_key, piece, g.n * pieces, bytes);
+    if (c < cost) {
+      cost = c;
+      best = KvPlan{g.n * pieces, pieces, piece};
+    }
+  }
+  return best;
+}
+
+// The forward's and dQ's chunk table: the chunks in ring order, each as its
+// plan's pieces (a piece past a chunk's valid keys is empty).
+void fill_kv_table(ChunkTable* ct, const KvPlan& kp, const Geometry& g, const void* const* k_chunks,
+                   const void* const* v_chunks, int64_t row_stride, int ring_rank) {
+  ct->n = g.n * kp.pieces;
+  for (int s = 0; s < g.n; ++s) {
+    const int c = (s + ring_rank) % g.n;
+    for (int j = 0; j < kp.pieces; ++j) {
+      const int i = s * kp.pieces + j, start = j * kp.piece;
+      const int left = g.len[c] > start ? g.len[c] - start : 0;
+      const int64_t off = left ? start * row_stride : 0;
+      ct->k[i] = static_cast<const bf16*>(k_chunks[c]) + off;
+      ct->v[i] = static_cast<const bf16*>(v_chunks[c]) + off;
+      ct->len[i] = kp.pieces > 1 && left > kp.piece ? kp.piece : left;
+      ct->order[i] = i;
+    }
+  }
+}
+
+// Query splits of the dK/dV kernel (with dQ's key pieces: backward of 8 heads x
+// 1500 x 1500 111 -> 82 us at head dim 128, 74 -> 53 at 64; x 4096 x 4096 268
+// -> 241).
+struct QPlan {
+  int n_split;
+  int rows;  // queries per split, a multiple of 64
+};
+QPlan q_plan(int batch, int h_num, int t_num, int h_len, int kv_chunk_len, int n_chunks) {
+  QPlan best{1, (t_num + 63) / 64 * 64};
+  const int fill =
+      grid_fill((int64_t)((kv_chunk_len + kDkdvBlockKeys - 1) / kDkdvBlockKeys) * n_chunks * h_num * batch);
+  const double bytes = 16. * batch * h_num * n_chunks * kv_chunk_len * h_len;  // dK and dV partials
+  double cost = split_cost(kDkdvUsPerQuery, t_num, 1, bytes);
+  for (int n = 2; n <= fill && n <= kMaxQSplits && n <= t_num / kMinStream; ++n) {
+    const int rows = ((t_num + n - 1) / n + 63) / 64 * 64, splits = (t_num + rows - 1) / rows;
+    const double c = split_cost(kDkdvUsPerQuery, rows, splits, bytes);
+    if (c < cost) {
+      cost = c;
+      best = QPlan{splits, rows};
+    }
+  }
+  return best;
 }
 
 // Forward: no scratch, except the KV splits' partial O (fp32 [n][B,H,T,D])
 // and row statistics (fp32 m and l, [n][B,H,T] each).
 struct FwdLayout {
-  int n_split;
+  KvPlan kv;
   size_t o, m, l, bytes;  // byte offsets
 };
 FwdLayout fwd_layout(int batch, int h_num, int t_num, int h_len, const Geometry& g) {
-  FwdLayout w{kv_splits(batch, h_num, t_num, g), 0, 0, 0, 0};
-  if (w.n_split < 2) return w;
+  FwdLayout w{kv_plan(kFwdUsPerKey, batch, h_num, t_num, h_len, g), 0, 0, 0, 0};
+  if (w.kv.n_split < 2) return w;
   const size_t rows = (size_t)batch * h_num * t_num;
-  w.m = round256(sizeof(float) * w.n_split * rows * h_len);
-  w.l = w.m + round256(sizeof(float) * w.n_split * rows);
-  w.bytes = w.l + round256(sizeof(float) * w.n_split * rows);
+  w.m = round256(sizeof(float) * w.kv.n_split * rows * h_len);
+  w.l = w.m + round256(sizeof(float) * w.kv.n_split * rows);
+  w.bytes = w.l + round256(sizeof(float) * w.kv.n_split * rows);
   return w;
 }
 size_t fwd_ws(int batch, int h_num, int t_num, int h_len, const Geometry& g) {
@@ -203,20 +306,28 @@ size_t fwd_ws(int batch, int h_num, int t_num, int h_len, const Geometry& g) {
 
 // Backward: the per-query statistics, written once per call by the dQ
 // kernel for the dK/dV kernel, in two fp32 planes of B*H*T rows; then, with
-// KV splits, the dQ kernel's partials (fp32 [n][B,H,T,D]).
+// KV splits, the dQ kernel's partials (fp32 [n][B,H,T,D]), or, with query
+// splits, the dK/dV kernel's (fp32 [n][B,H,N*Tc,D] of dK, then of dV), in the
+// same place: the dQ partials are merged before the dK/dV kernel starts.
 struct BwdLayout {
-  int n_split;
-  size_t stats, dq, bytes;  // byte offsets
+  KvPlan kv;
+  QPlan q;
+  size_t stats, dq, dk, dv, bytes;  // byte offsets
 };
-BwdLayout bwd_layout(int batch, int h_num, int t_num, int h_len, const Geometry& g) {
-  BwdLayout w{kv_splits(batch, h_num, t_num, g), 0, 0, 0};
-  const size_t rows = (size_t)batch * h_num * t_num;
-  w.dq = round256(2 * sizeof(float) * rows);
-  w.bytes = w.dq + (w.n_split > 1 ? round256(sizeof(float) * w.n_split * rows * h_len) : 0);
+BwdLayout bwd_layout(int batch, int h_num, int t_num, int h_len, int kv_chunk_len, const Geometry& g) {
+  BwdLayout w{kv_plan(kDqUsPerKey, batch, h_num, t_num, h_len, g), q_plan(batch, h_num, t_num, h_len, kv_chunk_len, g.n), 0, 0, 0, 0, 0};
+  const size_t rows = (size_t)batch * h_num * t_num, keys = (size_t)batch * h_num * g.n * kv_chunk_len;
+  w.dq = w.dk = w.dv = w.bytes = round256(2 * sizeof(float) * rows);
+  if (w.kv.n_split > 1) w.bytes = w.dq + round256(sizeof(float) * w.kv.n_split * rows * h_len);
+  if (w.q.n_split > 1) {
+    w.dv = w.dk + round256(sizeof(float) * w.q.n_split * keys * h_len);
+    const size_t end = w.dv + (w.dv - w.dk);
+    w.bytes = end > w.bytes ? end : w.bytes;
+  }
   return w;
 }
-size_t bwd_ws(int batch, int h_num, int t_num, int h_len, const Geometry& g) {
-  return bwd_layout(batch, h_num, t_num, h_len, g).bytes;
+size_t bwd_ws(int batch, int h_num, int t_num, int h_len, int kv_chunk_len, const Geometry& g) {
+  return bwd_layout(batch, h_num, t_num, h_len, kv_chunk_len, g).bytes;
 }
 
 // Library-owned grow-only workspace, one per device (used when the caller
@@ -373,24 +484,18 @@ int forward_impl(const void* q, const int64_t* q_strides, const void* const* k_c
   p.T = t_num;
   p.D = h_len;
   p.scale = scale;
-  p.ct.n = sp_size;
-  for (int c = 0; c < sp_size; ++c) {
-    p.ct.k[c] = static_cast<const bf16*>(k_chunks[c]);
-    p.ct.v[c] = static_cast<const bf16*>(v_chunks[c]);
-    p.ct.len[c] = g.len[c];
-    p.ct.order[c] = (c + ring_rank) % sp_size;
-  }
-  p.n_split = wl.n_split;
+  fill_kv_table(&p.ct, wl.kv, g, k_chunks, v_chunks, kv_strides[2], ring_rank);
+  p.n_split = wl.kv.n_split;
   FwdMergeParams mp;
   std::memset(&mp, 0, sizeof(mp));
-  if (wl.n_split > 1) {
+  if (wl.kv.n_split > 1) {
     // the kernel writes per-split partials (fp32, [n][B,H,T,D] and [n][B,H,T]);
     // the merge writes out / m_i / l_i
     char* ws = static_cast<char*>(workspace);
     mp.part_o = reinterpret_cast<const float*>(ws + wl.o);
     mp.part_m = reinterpret_cast<const float*>(ws + wl.m);
     mp.part_l = reinterpret_cast<const float*>(ws + wl.l);
-    mp.n_split = wl.n_split;
+    mp.n_split = wl.kv.n_split;
     mp.out = out;
     mp.sob = p.sob;
     mp.soh = p.soh;
@@ -420,7 +525,7 @@ int forward_impl(const void* q, const int64_t* q_strides, const void* const* k_c
   {
     TimedLaunch tl(HARP_RA_KERNEL_FWD, st);  // the merge is timed with the forward
     if ((rc = launched(launch_fwd(p, st), "forward"))) return rc;
-    if (wl.n_split > 1 && (rc = launched(launch_fwd_merge(mp, st), "forward merge"))) return rc;
+    if (wl.kv.n_split > 1 && (rc = launched(launch_fwd_merge(mp, st), "forward merge"))) return rc;
   }
   return ok();
 }
@@ -482,7 +587,7 @@ int backward_impl(const void* q, const int64_t* q_strides, void* grad_q, const i
   if (!delta && (rc = check_plain_view(out, out_strides, "out"))) return rc;
   if (m_i_dtype != HARP_RA_F32 && m_i_dtype != HARP_RA_BF16) return fail(HARP_RA_EINVAL, "m_i_dtype must be F32 or BF16");
 
-  const BwdLayout wl = bwd_layout(batch, h_num, t_num, h_len, g);
+  const BwdLayout wl = bwd_layout(batch, h_num, t_num, h_len, kv_chunk_len, g);
   if ((rc = resolve_workspace(&workspace, &workspace_bytes, wl.bytes))) return rc;
   hipStream_t st = static_cast<hipStream_t>(stream);
 
@@ -545,12 +650,13 @@ int backward_impl(const void* q, const int64_t* q_strides, void* grad_q, const i
   p.n_split = 1;
   // dQ first: it writes the per-query statistics planes the dK/dV kernel reads
   BwdParams pk = p;
+  fill_kv_table(&p.ct, wl.kv, g, k_chunks, v_chunks, kv_strides[2], ring_rank);
   DqMergeParams mp;
   std::memset(&mp, 0, sizeof(mp));
-  if (wl.n_split > 1) {
+  if (wl.kv.n_split > 1) {
     // per-split fp32 partials [n][B,H,T,D], summed into grad_q by the merge
     mp.part = reinterpret_cast<const float*>(ws + wl.dq);
-    mp.n_split = wl.n_split;
+    mp.n_split = wl.kv.n_split;
     mp.dq = grad_q;
     mp.sdqb = p.sdqb;
     mp.sdqh = p.sdqh;
@@ -560,7 +666,7 @@ int backward_impl(const void* q, const int64_t* q_strides, void* grad_q, const i
     mp.H = h_num;
     mp.T = t_num;
     mp.D = h_len;
-    p.n_split = wl.n_split;
+    p.n_split = wl.kv.n_split;
     p.dq = ws + wl.dq;
     p.dq_f32 = 1;
     p.sdqt = h_len;
@@ -571,11 +677,45 @@ int backward_impl(const void* q, const int64_t* q_strides, void* grad_q, const i
   {
     TimedLaunch tl(HARP_RA_KERNEL_DQ, st);  // the merge is timed with the dQ kernel
     if ((rc = launched(launch_dq(p, st), "dQ"))) return rc;
-    if (wl.n_split > 1 && (rc = launched(launch_dq_merge(mp, st), "dQ merge"))) return rc;
+    if (wl.kv.n_split > 1 && (rc = launched(launch_dq_merge(mp, st), "dQ merge"))) return rc;
+  }
+  pk.q_rows = wl.q.rows;
+  pk.n_split = wl.q.n_split;
+  DkdvMergeParams kp;
+  std::memset(&kp, 0, sizeof(kp));
+  if (wl.q.n_split > 1) {
+    // per-split fp32 partials [n][B,H,N*Tc,D], summed into the chunks' dK / dV by the merge
+    const int64_t keys = (int64_t)sp_size * kv_chunk_len;
+    kp.part_dk = reinterpret_cast<const float*>(ws + wl.dk);
+    kp.part_dv = reinterpret_cast<const float*>(ws + wl.dv);
+    kp.n_split = wl.q.n_split;
+    kp.dkv_f32 = pk.dkv_f32;
+    kp.wide = !pk.dkv_f32 && ((pk.sdkb | pk.sdkh | pk.sdkt) & 3) == 0;
+    kp.sdkb = pk.sdkb;
+    kp.sdkh = pk.sdkh;
+    kp.sdkt = pk.sdkt;
+    kp.B = batch;
+    kp.H = h_num;
+    kp.D = h_len;
+    kp.n_chunks = sp_size;
+    kp.chunk_len = kv_chunk_len;
+    for (int c = 0; c < sp_size; ++c) {
+      kp.dk[c] = pk.ct.dk[c];
+      kp.dv[c] = pk.ct.dv[c];
+      if (((reinterpret_cast<uintptr_t>(kp.dk[c]) | reinterpret_cast<uintptr_t>(kp.dv[c])) & 7u) != 0) kp.wide = 0;
+      pk.ct.dk[c] = reinterpret_cast<bf16*>(reinterpret_cast<float*>(ws + wl.dk) + (int64_t)c * kv_chunk_len * h_len);
+      pk.ct.dv[c] = reinterpret_cast<bf16*>(reinterpret_cast<float*>(ws + wl.dv) + (int64_t)c * kv_chunk_len * h_len);
+    }
+    pk.dkv_f32 = 1;
+    pk.sdkt = h_len;
+    pk.sdkh = keys * h_len;
+    pk.sdkb = h_num * pk.sdkh;
+    pk.split_dkv = batch * pk.sdkb;
   }
   {
-    TimedLaunch tl(HARP_RA_KERNEL_DKDV, st);
+    TimedLaunch tl(HARP_RA_KERNEL_DKDV, st);  // the merge is timed with the dK/dV kernel
     if ((rc = launched(launch_dkdv(pk, st), "dK/dV"))) return rc;
+    if (wl.q.n_split > 1 && (rc = launched(launch_dkdv_merge(kp, st), "dK/dV merge"))) return rc;
   }
   return ok();
 }
@@ -629,7 +769,7 @@ size_t harp_ra_backward_workspace_bytes(int batch, int h_num, int t_num, int h_l
   Geometry g;
   if (check_dims(batch, h_num, t_num, h_len) != HARP_RA_OK) return SIZE_MAX;
   if (make_geometry(sp_size, kv_chunk_len, kv_valid_lens, &g) != HARP_RA_OK) return SIZE_MAX;
-  return bwd_ws(batch, h_num, t_num, h_len, g);
+  return bwd_ws(batch, h_num, t_num, h_len, kv_chunk_len, g);
 }
 
 int harp_ra_forward(const void* q, const int64_t* q_strides, const void* const* k_chunks,

@@ -55,6 +55,20 @@ struct DqMergeParams {
   int B, H, T, D;
 };
 
+// Sums the query splits' dK and dV partials (fp32, dK already scaled, pad
+// keys zero, [n][B,H,N*Tc,D] each) into the chunks' views.
+struct DkdvMergeParams {
+  const float* part_dk;
+  const float* part_dv;
+  int n_split;
+  bf16* dk[kMaxChunks];
+  bf16* dv[kMaxChunks];
+  int64_t sdkb, sdkh, sdkt;
+  int dkv_f32;
+  int wide;  // bf16 rows 8-byte aligned
+  int B, H, D, n_chunks, chunk_len;
+};
+
 struct DeltaParams {
   const bf16* dout;
   int64_t sdb, sdh, sdt;
@@ -82,8 +96,10 @@ struct BwdParams {
   const float* out;            // the forward's fp32 O (read only when delta is NULL)
   int64_t sob, soh, sot;
   float* stats;             // workspace [2][B*H*T]: -(m + ln l) / scale, -D (written by the dQ kernel)
-  int n_split;              // KV splits of the dQ kernel (grid dimension y); > 1: dq is per-split partials
+  int n_split;              // grid dimension y: KV splits (dQ) or query splits (dK/dV); > 1: partial outputs
   int64_t split_dq;         // elements between the splits' dQ buffers
+  int q_rows;               // dK/dV: queries per split
+  int64_t split_dkv;        // elements between the splits' dK (dV) buffers
   int n_key_tiles;          // kDkdvBlockKeys-key blocks per (b, h) over all chunks
   int ct_rows[kMaxChunks];  // stored rows of chunk c (dK/dV rows written, pads get 0)
   int B, H, T, D;
@@ -102,6 +118,17 @@ __device__ __forceinline__ float bwd_stat_lse(const BwdParams& p, int64_t i) {
   return (ll > 0.f) ? -(mm + __logf(ll)) * p.inv_scale : -INFINITY;
 }
 
+// The dK/dV kernels' query split (grid dimension y): queries begin ..
+// begin + rows - 1, never none.
+struct QSplit {
+  int64_t begin;
+  int rows;
+};
+__device__ __forceinline__ QSplit q_split(const BwdParams& p) {
+  const int begin = (int)blockIdx.y * p.q_rows, left = p.T - begin;
+  return QSplit{begin, left < p.q_rows ? left : p.q_rows};
+}
+
 // Keys per dK/dV block (the host sizes the grid and the chunk table with it).
 constexpr int kDkdvBlockKeys = 256;
 
@@ -112,6 +139,7 @@ bool fwd_asm_applies(const FwdParams& p);
 hipError_t launch_fwd_asm(const FwdParams& p, hipStream_t st);
 hipError_t launch_fwd_merge(const FwdMergeParams& p, hipStream_t st);
 hipError_t launch_dq_merge(const DqMergeParams& p, hipStream_t st);
+hipError_t launch_dkdv_merge(const DkdvMergeParams& p, hipStream_t st);
 // Query rows per block of the forward and dQ kernels (the host sizes KV splits with it).
 constexpr int kQueryBlockRows = 256;
 hipError_t launch_delta(const DeltaParams& p, hipStream_t st);

@@ -1156,9 +1156,10 @@ __global__ __launch_bounds__(64 * kDkWaves, 1) void dkdv_kernel(BwdParams p) {
     DirectLoader<GQ, kDkWaves> qld, gld;
     qld.init(p.sqt, p.D, wave, lane);
     gld.init(p.sdt, p.D, wave, lane);
-    const bf16* qb_ = p.q + (int64_t)b * p.sqb + (int64_t)h * p.sqh;
-    const bf16* gb_ = p.dout + (int64_t)b * p.sdb + (int64_t)h * p.sdh;
-    const int64_t sbase = ((int64_t)b * p.H + h) * p.T;
+    const QSplit qs = q_split(p);
+    const bf16* qb_ = p.q + (int64_t)b * p.sqb + (int64_t)h * p.sqh + qs.begin * p.sqt;
+    const bf16* gb_ = p.dout + (int64_t)b * p.sdb + (int64_t)h * p.sdh + qs.begin * p.sdt;
+    const int64_t sbase = ((int64_t)b * p.H + h) * p.T + qs.begin;
     const int64_t nrows = (int64_t)p.B * p.H * p.T;
 
     // Per-query statistics of a tile (the two prepared planes, 64 rows each)
@@ -1169,14 +1170,14 @@ __global__ __launch_bounds__(64 * kDkWaves, 1) void dkdv_kernel(BwdParams p) {
         const uint32_t voff = (uint32_t)lane * 4u;
 #pragma unroll
         for (int pl = 0; pl < 2; ++pl) {
-          const rsrc_t rs = make_rsrc(p.stats + pl * nrows + sbase + q0, (uint32_t)(p.T - q0) * 4u);
+          const rsrc_t rs = make_rsrc(p.stats + pl * nrows + sbase + q0, (uint32_t)(qs.rows - q0) * 4u);
           lds_dma_b32(rs, (uint32_t)(uintptr_t)(lds_void*)&St[bf][pl][0], voff);
         }
       }
     };
     auto issue = [&](int q0, int bf) {
-      qld.load(rows_rsrc(qb_, p.sqt, q0, p.T - q0), QG[bf][0]);
-      gld.load(rows_rsrc(gb_, p.sdt, q0, p.T - q0), QG[bf][1]);
+      qld.load(rows_rsrc(qb_, p.sqt, q0, qs.rows - q0), QG[bf][0]);
+      gld.load(rows_rsrc(gb_, p.sdt, q0, qs.rows - q0), QG[bf][1]);
       issue_stats(q0, bf);
     };
     // Inside the loop the next tile's copies are issued one instruction per
@@ -1234,7 +1235,7 @@ __global__ __launch_bounds__(64 * kDkWaves, 1) void dkdv_kernel(BwdParams p) {
       }
       return x;
     };
-    const int n_tiles = (p.T + 63) >> 6;
+    const int n_tiles = (qs.rows + 63) >> 6;
     int buf = 0;
 #pragma unroll 1
     for (int t = 0; t < n_tiles; ++t) {
@@ -1243,8 +1244,8 @@ __global__ __launch_bounds__(64 * kDkWaves, 1) void dkdv_kernel(BwdParams p) {
       const bool has_next = t + 1 < n_tiles;
       const int nq0 = (t + 1) * 64;
       if (has_next) {
-        nq_rs = rows_rsrc(qb_, p.sqt, nq0, p.T - nq0);
-        ng_rs = rows_rsrc(gb_, p.sdt, nq0, p.T - nq0);
+        nq_rs = rows_rsrc(qb_, p.sqt, nq0, qs.rows - nq0);
+        ng_rs = rows_rsrc(gb_, p.sdt, nq0, qs.rows - nq0);
       }
       const bf16* Q = QG[buf][0];
       const bf16* Gd = QG[buf][1];
@@ -1316,7 +1317,7 @@ __global__ __launch_bounds__(64 * kDkWaves, 1) void dkdv_kernel(BwdParams p) {
 
   // store: C layout row = key key0 + c_row(r,g), col = d = db*32 + l32;
   // keys past the valid length (pads) get zero
-  const int64_t base = (int64_t)b * p.sdkb + (int64_t)h * p.sdkh;
+  const int64_t base = (int64_t)b * p.sdkb + (int64_t)h * p.sdkh + (int64_t)blockIdx.y * p.split_dkv;
   const int lane_e = lane_id_fresh(), g_e = lane_e >> 5;  // as in the forward's epilogue
   using E = cq_epi::KRows<DPE>;
   if constexpr (E::kHalfBytes <= (int)sizeof(QG) && E::kHalfBytes <= (int)sizeof(Vb)) {
@@ -1532,6 +1533,52 @@ __global__ __launch_bounds__(256) void dq_merge_kernel(DqMergeParams p) {
   }
 }
 
+// One pass over the partial dK and dV: LPR lanes per key row, 8 elements of D
+// per lane, all splits' loads of a tensor in flight together (at most 8).
+template <int LPR>
+__global__ __launch_bounds__(256) void dkdv_merge_kernel(DkdvMergeParams p) {
+  const int64_t L = (int64_t)p.n_chunks * p.chunk_len, rows = (int64_t)p.B * p.H * L;
+  const int64_t row = (int64_t)blockIdx.x * (256 / LPR) + (threadIdx.x / LPR);
+  const int d0 = (threadIdx.x % LPR) * 8;
+  if (row >= rows || d0 >= p.D) return;
+  const int64_t bh = row / L;
+  const int key = (int)(row - bh * L), c = key / p.chunk_len, t = key - c * p.chunk_len;
+  const int h = (int)(bh % p.H), b = (int)(bh / p.H);
+  const int64_t e = (int64_t)b * p.sdkb + (int64_t)h * p.sdkh + (int64_t)t * p.sdkt + d0;
+#pragma unroll
+  for (int tn = 0; tn < 2; ++tn) {
+    const float* part = (tn == 0 ? p.part_dk : p.part_dv) + row * p.D + d0;
+    f32x4 x[8], y[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {  // an index past the last split reads the last one again, unused
+      const float* s = part + min(u, p.n_split - 1) * rows * p.D;
+      x[u] = *(const f32x4*)s;
+      y[u] = *(const f32x4*)(s + 4);
+    }
+    f32x4 ax = x[0], ay = y[0];
+#pragma unroll
+    for (int u = 1; u < 8; ++u) {
+      if (u >= p.n_split) break;
+      ax += x[u];
+      ay += y[u];
+    }
+    bf16* const o = tn == 0 ? p.dk[c] : p.dv[c];
+    if (p.dkv_f32) {
+      *(f32x4u*)((float*)o + e) = ax;
+      *(f32x4u*)((float*)o + e + 4) = ay;
+    } else if (p.wide) {
+      *(bf16x4*)(o + e) = __builtin_convertvector(ax, bf16x4);
+      *(bf16x4*)(o + e + 4) = __builtin_convertvector(ay, bf16x4);
+    } else {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        o[e + j] = (bf16)ax[j];
+        o[e + 4 + j] = (bf16)ay[j];
+      }
+    }
+  }
+}
+
 namespace {
 
 // The merge instance for this split count and head dim: group = splits (2..8;
@@ -1573,6 +1620,15 @@ struct DqMergeK {
 
 hipError_t launch_fwd_merge(const FwdMergeParams& p, hipStream_t st) { return launch_merge<FwdMergeK>(p, st); }
 hipError_t launch_dq_merge(const DqMergeParams& p, hipStream_t st) { return launch_merge<DqMergeK>(p, st); }
+hipError_t launch_dkdv_merge(const DkdvMergeParams& p, hipStream_t st) {
+  const int64_t rows = (int64_t)p.B * p.H * p.n_chunks * p.chunk_len;
+  const bool narrow = p.D <= 64;
+  const int rpb = narrow ? 32 : 16;
+  const dim3 grid((unsigned)((rows + rpb - 1) / rpb)), block(256);
+  if (narrow) hipLaunchKernelGGL(dkdv_merge_kernel<8>, grid, block, 0, st, p);
+  else hipLaunchKernelGGL(dkdv_merge_kernel<16>, grid, block, 0, st, p);
+  return hipGetLastError();
+}
 
 // Every (KSTEPS, DBLK) variant the launchers dispatch to, instantiated
 // explicitly: with lambdas in the kernel bodies the host pass otherwise
@@ -1606,7 +1662,7 @@ static hipError_t launch_dq_t(const BwdParams& p, hipStream_t st) {
 template <int KSTEPS, int DBLK>
 static hipError_t launch_dkdv_t(const BwdParams& p, hipStream_t st) {
   const int n = p.n_key_tiles * p.H * p.B;
-  hipLaunchKernelGGL((dkdv_kernel<KSTEPS, DBLK>), dim3(n), dim3(64 * kDkWaves), 0, st, p);
+  hipLaunchKernelGGL((dkdv_kernel<KSTEPS, DBLK>), dim3(n, p.n_split), dim3(64 * kDkWaves), 0, st, p);
   return hipGetLastError();
 }
 

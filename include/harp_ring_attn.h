@@ -164,13 +164,14 @@ HARP_RA_API int harp_ra_delta(const void* grad_out, const int64_t* do_strides,
  * current device ((size_t)-1 when the arguments are invalid; 0 = none
  * needed).  The forward keeps all staging in LDS; the backward needs 8 bytes
  * per query row (B*H*T, rounded up to 256 bytes) for its per-query
- * statistics, prepared once per call.  When the forward / dQ grids would
- * leave at least half of the device's compute units idle (fewer than
- * CUs / 2 tiles of 256 queries over B and H) and there are several chunks,
- * the ring steps are split over up to sp_size blocks per tile: the forward
- * then needs n * B*H*T * (4*h_len + 8) bytes for the splits' partial O, m
- * and l, and the backward n * B*H*T * 4*h_len more for the dQ partials (each
- * part rounded up to 256 bytes).  Replaces the reference's grow-only scratch sizing
+ * statistics, prepared once per call.  When a grid would leave at least half
+ * of the device's compute units idle (fewer than CUs / 2 tiles of 256 queries,
+ * for dK / dV of 256 keys, over B and H), its blocks' keys (queries) may be
+ * split over n blocks each, where that is estimated to pay: the forward then
+ * needs n * B*H*T * (4*h_len + 8) bytes for the splits' partial O, m and l
+ * (n <= 16), and the backward the larger of n * B*H*T * 4*h_len for the dQ
+ * partials and n * B*H*sp_size*kv_chunk_len * 8*h_len (n <= 8) for the dK and
+ * dV partials (each part rounded up to 256 bytes).  Replaces the reference's grow-only scratch sizing
  * (RingAttnHbmWorkspace::ensure_slot, ring_attn.cpp:620-840, sized at
  * :2428-2450 and :2595-2656).
  */

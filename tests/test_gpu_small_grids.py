@@ -1,0 +1,84 @@
+"""GPU: calls whose grids leave most CUs idle, where the forward and dQ split
+the keys of a chunk (not only the ring steps) and dK/dV splits the queries,
+against fp64 attention: piece edges, pad keys that leave pieces empty, several
+chunks in rotated ring order, bf16 and fp32 gradients, unaligned bf16 views."""
+
+import math
+
+import pytest
+import torch
+
+import harp_amd
+from harp_amd import ops as H_ops
+
+pytestmark = pytest.mark.gpu
+
+DEV = "cuda:0"
+
+# (B, H, T, D, sp, chunk, valid per chunk, ring_rank)
+SHAPES = [
+    (1, 3, 1000, 128, 1, 1000, [1000], 0), (1, 2, 511, 128, 1, 4096, [4000], 0), (1, 2, 513, 128, 3, 700, [700, 129, 0], 1),
+    (2, 1, 2049, 128, 2, 513, [513, 257], 1), (1, 3, 1000, 64, 1, 1000, [999], 0), (1, 2, 576, 64, 3, 600, [600, 1, 300], 2),
+    (1, 2, 700, 72, 2, 1030, [1030, 512], 0), (1, 2, 640, 96, 1, 900, [900], 0), (1, 1, 2000, 40, 2, 520, [520, 520], 1),
+]
+
+
+def _ref(q, k, v, dout, keep):
+    q, k, v, dout = (t.double() for t in (q, k[:, :, keep], v[:, :, keep], dout))
+    scale = 1.0 / math.sqrt(q.shape[-1])
+    s = torch.matmul(q, k.transpose(-1, -2).contiguous()) * scale
+    p = torch.softmax(s, -1)
+    o = torch.matmul(p, v)
+    ds = p * (torch.matmul(dout, v.transpose(-1, -2).contiguous()) - (dout * o).sum(-1, keepdim=True)) * scale
+    return (o, torch.matmul(ds, k), torch.matmul(ds.transpose(-1, -2).contiguous(), q),
+            torch.matmul(p.transpose(-1, -2).contiguous(), dout), torch.logsumexp(s, -1))
+
+
+def _rel(a, b):
+    return float((a.double() - b).norm() / b.norm())
+
+
+@pytest.mark.parametrize("B,H,T,D,sp,chunk,lens,rank", SHAPES)
+@pytest.mark.parametrize("grads", ["bf16", "fp32", "bf16 unaligned"])
+def test_split_calls_against_fp64(B, H, T, D, sp, chunk, lens, rank, grads):
+    if grads == "bf16 unaligned" and D == 128:
+        pytest.skip("head dim 128 stores bf16 gradients 8 bytes at a time: the C ABI refuses such views")
+    g = torch.Generator(device=DEV).manual_seed(T + D)
+    q, dout = (torch.randn(B, T, H, D, device=DEV, generator=g).to(torch.bfloat16).transpose(1, 2) for _ in range(2))
+    k, v = (torch.randn(B, sp * chunk, H, D, device=DEV, generator=g).to(torch.bfloat16).transpose(1, 2) for _ in range(2))
+    pos = torch.arange(sp * chunk, device=DEV)
+    keep = (pos % chunk) < torch.tensor(lens, device=DEV)[pos // chunk]
+    o64, dq64, dk64, dv64, lse64 = _ref(q, k, v, dout, keep)
+    scale = 1.0 / math.sqrt(D)
+    kc = [k[:, :, c * chunk:(c + 1) * chunk] for c in range(sp)]
+    vc = [v[:, :, c * chunk:(c + 1) * chunk] for c in range(sp)]
+    out, m, l = torch.empty_like(q, dtype=torch.float32), torch.empty(B, H, T, device=DEV), torch.empty(B, H, T, device=DEV)
+    H_ops.abi_forward(q, kc, vc, out, m, l, scale, rank, lens)
+    delta = torch.empty(B, H, T, device=DEV)
+    H_ops.abi_delta(dout, out, delta)
+    dt = torch.float32 if grads == "fp32" else torch.bfloat16
+    pad = 1 if "unaligned" in grads else 0  # rows start on odd elements
+    mk = lambda n: torch.full((B, n, H, D + pad), float("nan"), device=DEV, dtype=dt)[..., pad:].transpose(1, 2)  # noqa: E731
+    dq, dk, dv = mk(T), mk(sp * chunk), mk(sp * chunk)
+    ch = lambda t: [t[:, :, c * chunk:(c + 1) * chunk] for c in range(sp)]  # noqa: E731
+    H_ops.abi_backward(q, dq, kc, vc, ch(dk), ch(dv), dout, m, l, delta, scale, rank, lens)
+    assert float((m.double() + l.double().log() - lse64).abs().max()) <= 1e-4
+    # P, dS and (bf16 outputs) the results are rounded to bf16, 2^-9 rms each:
+    # at most three such roundings reach a result
+    for name, a, b in (("o", out, o64), ("dq", dq, dq64), ("dk", dk[:, :, keep], dk64), ("dv", dv[:, :, keep], dv64)):
+        assert _rel(a, b) <= 3 * 2.0 ** -9, (name, _rel(a, b))
+    assert not dk[:, :, ~keep].any() and not dv[:, :, ~keep].any()
+
+
+def test_a_smaller_workspace_is_refused():
+    lib = harp_amd.load_abi()
+    need = H_ops.backward_workspace_bytes(1, 2, 1024, 128, 1, 1024)
+    assert need > 2 * 4 * 2 * 1024  # more than the statistics: split partials
+    g = torch.Generator(device=DEV).manual_seed(1)
+    q = torch.randn(1, 1024, 2, 128, device=DEV, generator=g).to(torch.bfloat16).transpose(1, 2)
+    f = torch.zeros(1, 2, 1024, device=DEV)
+    ws = torch.empty(need - 256, dtype=torch.uint8, device=DEV)
+    with pytest.raises(RuntimeError, match="workspace"):
+        H_ops.abi_backward(q, torch.empty_like(q), [q], [q], [torch.empty_like(q)], [torch.empty_like(q)], q, f, f, f,
+                           1.0, workspace=ws)
+    assert "smaller" in lib.harp_ra_last_error().decode()

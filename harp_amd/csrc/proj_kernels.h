@@ -9,8 +9,8 @@
 namespace harp_proj {
 
 constexpr int kHeadDim = 128;       // features of one head (one wave's share)
-constexpr int kBlockHeads = 2;      // heads per block
-constexpr int kBlockTokens = 256;   // tokens per block
+constexpr int kBlockHeads = 2;      // heads per unit of the large grid
+constexpr int kBlockTokens = 256;   // tokens per unit of the large grid
 constexpr int kKTile = 64;        // contraction elements per LDS tile
 constexpr int kMaxOuts = 3;       // q, k, v in one launch
 
@@ -42,8 +42,10 @@ struct ProjParams {
   int n_lin, keep_last, tail_bid0;
 };
 
-// LDS bytes of the main kernel: two stages of the x and W tiles
-constexpr int kProjLdsBytes = 2 * (kBlockTokens + kBlockHeads * kHeadDim) * kKTile * 2;
+// LDS bytes the tiles of one block may take: two stages of the 256-token x
+// 2-head x and W tiles, or three or four of the smaller blocks' tiles, beside
+// the norm weight in the CU's 160 KB
+constexpr int kProjLdsBytes = 144 * 1024;
 
 hipError_t launch_proj(const ProjParams& p, hipStream_t stream);
 

@@ -32,16 +32,23 @@
 //            needs no exchange between waves;
 //   k-tile = 64 elements: x tile 256 x 64 and W tile 256 x 64 (32 KB each),
 //            copied global -> LDS by buffer_load ... lds into two stages.
-// Work units are 256-token x 2-head tiles.  When they leave the last round of
-// the CUs at most half full (1152 units on 256 CUs at the headline shape: 4.5
-// rounds), the units of that round run in a second launch as two 128-token
-// halves each (the same kernel with 32 tokens per wave), which fill one round
-// at half the time, instead of half the CUs idling through a whole one.
+// These blocks are MFMA- and LDS-bound and the fastest per token once the CUs
+// are full (386 us, 1200 TFLOP/s, at 8192 tokens x 24 heads x 3).  Two smaller
+// ones, bit for bit the same arithmetic, serve grids that leave CUs idle and
+// the last round of the CUs; there a tile's few MFMAs don't cover the memory's
+// latency with one tile of lead, so more stages are in flight:
+//   32 tokens per wave, 2 heads: 128 tokens x 2 heads, 48 KB a tile, three
+//            stages (two stages: 10-13 us slower at 256 tokens x 24 or 30 heads);
+//   32 tokens per wave, 1 head: 4 waves, 128 tokens x 1 head, 32 KB a tile,
+//            four stages.  At 256 tokens x 30 heads it fills 180 of the CUs
+//            where the large blocks fill 45, and reads the 88 MB of weights at
+//            2.5 TB/s: 83 -> 35 us.
+// launch_proj has the rule.
 // Pipeline: one barrier per tile, in its last k-step, after which nobody
 // reads tile t's stage any more (its last fragments are in registers) and
-// tile t + 1 is complete; the copies of tile t + 2 then go into tile t's
+// tile t + 1 is complete; the copies of tile t + stages then go into tile t's
 // stage, between the MFMAs of that last k-step, and have until the barrier
-// of the next tile to land.  Fragment reads run on across tile boundaries.
+// before their tile to land.  Fragment reads run on across tile boundaries.
 #include "proj_kernels.h"
 #include "ra_common.h"
 
@@ -58,20 +65,14 @@ using harp_ra::mfma32x32x16;
 using harp_ra::rsrc_t;
 using harp_ra::sched_fence;
 using harp_ra::wait_lds_loads;
+using harp_ra::wait_lds_loads_but;
 using harp_ra::zero16;
 
 namespace {
 
-constexpr int kWaves = 8;
-constexpr int kStages = 2;
-constexpr int kFeatures = kBlockHeads * kHeadDim;     // 256
+constexpr int kTokenGroups = 4;                       // waves per head of a block, along the tokens
 constexpr int kRowBytes = kKTile * 2;                 // 128: one row of a tile
-constexpr int kWBytes = kFeatures * kRowBytes;        // 32 KB
-constexpr int kWPerWave = kWBytes / 1024 / kWaves;    // 1 KB copy instructions per wave and tile: 4
-constexpr int kHeadPairGroup = 4;  // head pairs per group of the block order
-static_assert(kWBytes % (1024 * kWaves) == 0, "copies split evenly");
-static_assert(kStages * (kBlockTokens * kRowBytes + kWBytes) == kProjLdsBytes, "LDS budget");
-static_assert(kWaves == 2 * (kBlockTokens / 64), "waves = heads x token groups of 64");
+constexpr int kHeadGroup = 4;  // blocks along the heads per group of the block order
 
 template <int I>
 struct Int {
@@ -114,65 +115,75 @@ struct Frags {
 
 }  // namespace
 
-// TPW tokens per wave (64: the main grid, 256-token blocks; 32: the tail,
-// 128-token halves of the last round's units)
-template <int TPW>
-__global__ __launch_bounds__(64 * kWaves, 1) void proj_kernel(ProjParams p) {
+// TPW tokens per wave, HEADS heads per block, STAGES tiles in LDS; TAIL: the
+// blocks are parts (of 128 tokens x HEADS heads) of the main grid's last units
+template <int TPW, int HEADS, int STAGES, bool TAIL>
+__global__ __launch_bounds__(64 * kTokenGroups * HEADS, 1) void proj_kernel(ProjParams p) {
+  constexpr int kWaves = kTokenGroups * HEADS;
+  constexpr int kFeatures = HEADS * kHeadDim;
+  constexpr int kWBytes = kFeatures * kRowBytes;          // 16 KB per head
+  constexpr int kWPerWave = kWBytes / 1024 / kWaves;      // 1 KB copy instructions per wave and tile: 4
   constexpr int NJ = TPW / 32;                            // 32-token blocks per wave
-  constexpr int kTok = 4 * TPW;                           // tokens per block
+  constexpr int kTok = kTokenGroups * TPW;                // tokens per block
   constexpr int kXBytes = kTok * kRowBytes;               // 32 or 16 KB
   constexpr int kXPerWave = kXBytes / 1024 / kWaves;      // 4 or 2
   constexpr int kDmaPerWave = kXPerWave + kWPerWave;      // 8 or 6 copies per tile
   constexpr int kMfma = 4 * NJ;                           // MFMAs per k-step
-  static_assert(kXBytes % (1024 * kWaves) == 0, "copies split evenly");
+  static_assert(kXBytes % (1024 * kWaves) == 0 && kWBytes % (1024 * kWaves) == 0, "copies split evenly");
+  static_assert(STAGES * (kXBytes + kWBytes) <= kProjLdsBytes, "LDS budget");
   // the stages: x tiles, then W tiles; after the main loop each wave's
   // TPW x 256 bytes serve as its staging rows for the output stores
-  __shared__ __attribute__((aligned(16))) char lds[kStages * (kXBytes + kWBytes)];
+  __shared__ __attribute__((aligned(16))) char lds[STAGES * (kXBytes + kWBytes)];
   __shared__ float norm_wf[kHeadDim];  // RMSNorm weight as fp32
-  static_assert(kWaves * TPW * 2 * kHeadDim <= kStages * (kXBytes + kWBytes), "staging fits the stages");
+  static_assert(kWaves * TPW * 2 * kHeadDim <= STAGES * (kXBytes + kWBytes), "staging fits the stages");
   auto Xs = [&](int s) { return lds + s * kXBytes; };
-  auto Ws = [&](int s) { return lds + kStages * kXBytes + s * kWBytes; };
+  auto Ws = [&](int s) { return lds + STAGES * kXBytes + s * kWBytes; };
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l32 = lane & 31, g = lane >> 5;
-  const int hh = wave & 1, tg = wave >> 1;  // head of the pair, token group (TPW)
+  const int hh = wave % HEADS, tg = wave / HEADS;  // head of the block, token group (TPW)
 
   // this block's unit (bid in the main grid's order) and output
-  int bid, y, half = 0;
-  if (TPW == 64) {
+  constexpr int kUnitHeads = TAIL ? kBlockHeads : HEADS;
+  constexpr int kUnitTok = TAIL ? kBlockTokens : kTok;
+  constexpr int kParts = (kUnitTok / kTok) * (kUnitHeads / HEADS);
+  int bid, y, part = 0;
+  if (!TAIL) {
     bid = (int)blockIdx.x;
     y = (int)blockIdx.y;
     if (y == p.n_outs - 1 && bid >= p.keep_last) return;  // left to the tail launch
   } else {
-    bid = p.tail_bid0 + (int)blockIdx.x / 2;
-    half = (int)blockIdx.x & 1;
+    bid = p.tail_bid0 + (int)blockIdx.x / kParts;
+    part = (int)blockIdx.x % kParts;
     y = p.n_outs - 1;
   }
 
   // block -> (token tile, head pair).  Workgroups are dealt to the 8 XCDs
   // round-robin; the remap gives each XCD a contiguous range of the order
-  // below, which walks groups of 4 head pairs, within a group the token
-  // tiles, and within a token tile the group's pairs.  The 32 blocks an XCD
-  // runs at once then cover 8 token tiles x 4 head pairs, and per k-tile read
-  // 12 tiles through its L2 (against 2 + 24 in token-tile-major order).
-  const int n_hp = (p.heads + kBlockHeads - 1) / kBlockHeads;
+  // below (the first total % 8 ranges are one longer), which walks groups of
+  // 4 head pairs, within a group the token tiles, and within a token tile the
+  // group's pairs.  The 32 blocks an XCD runs at once then cover 8 token
+  // tiles x 4 head pairs, and per k-tile read 12 tiles through its L2
+  // (against 2 + 24 in token-tile-major order).
+  const int n_hp = (p.heads + kUnitHeads - 1) / kUnitHeads;
   const int total = p.n_lin;
-  int lin = bid;
-  if (total % 8 == 0) lin = (lin % 8) * (total / 8) + lin / 8;
+  const int lin = (bid % 8) * (total / 8) + min(bid % 8, total % 8) + bid / 8;
   const int n_mt = total / n_hp;
-  const int grp = lin / (n_mt * kHeadPairGroup), gs = min(kHeadPairGroup, n_hp - grp * kHeadPairGroup);
-  const int rem = lin - grp * n_mt * kHeadPairGroup;
-  const int mt = rem / gs, hp = grp * kHeadPairGroup + rem % gs;
+  const int grp = lin / (n_mt * kHeadGroup), gs = min(kHeadGroup, n_hp - grp * kHeadGroup);
+  const int rem = lin - grp * n_mt * kHeadGroup;
+  const int mt = rem / gs, hp = grp * kHeadGroup + rem % gs;
   // (constant indices: a kernel-argument array indexed at run time would be
   // copied to scratch memory)
   const ProjOut o = y == 0 ? p.out[0] : (y == 1 ? p.out[1] : p.out[2]);
-  const int m0 = mt * kBlockTokens + half * kTok;
+  // parts of a unit: its token halves, then (one head per block) its heads
+  const int m0 = mt * kUnitTok + part % (kUnitTok / kTok) * kTok;
+  const int h0 = hp * kUnitHeads + part / (kUnitTok / kTok) * HEADS;
   const int rows_x = min(kTok, p.M - m0);
-  if (rows_x <= 0) return;  // the empty second half of a partial last token tile
-  const int rows_w = min(kFeatures, (p.heads - hp * kBlockHeads) * kHeadDim);  // an odd last head
+  if (rows_x <= 0 || h0 >= p.heads) return;  // a part past the last token or head
+  const int rows_w = min(kFeatures, (p.heads - h0) * kHeadDim);  // an odd last head
   const bf16* xb = (const bf16*)p.x + (int64_t)m0 * p.ldx;
-  const bf16* wb = (const bf16*)o.w + (int64_t)hp * kFeatures * o.ldw;
+  const bf16* wb = (const bf16*)o.w + (int64_t)h0 * kHeadDim * o.ldw;
   const uint32_t x_bytes = (uint32_t)((int64_t)rows_x * p.ldx * 2);
   const uint32_t w_bytes = (uint32_t)((int64_t)rows_w * o.ldw * 2);
 
@@ -194,16 +205,16 @@ __global__ __launch_bounds__(64 * kWaves, 1) void proj_kernel(ProjParams p) {
     const int k0 = t * kKTile;
     return make_rsrc(wb + k0, live ? w_bytes - (uint32_t)k0 * 2 : 0u);
   };
-  // copy j (0 .. kDmaPerWave - 1) of a tile into stage s
-  auto dma = [&](const rsrc_t& xr, const rsrc_t& wr, int s, int j) {
-    if (j < kXPerWave) {
-      const uint32_t dst = (uint32_t)(uintptr_t)(lds_void*)(Xs(s) + (wave + kWaves * j) * 1024);
-      lds_dma_b128(xr, __builtin_amdgcn_readfirstlane(dst), xsrc[j]);
-    } else {
-      const uint32_t dst =
-          (uint32_t)(uintptr_t)(lds_void*)(Ws(s) + (wave + kWaves * (j - kXPerWave)) * 1024);
-      lds_dma_b128(wr, __builtin_amdgcn_readfirstlane(dst), wsrc[j - kXPerWave]);
-    }
+  // copy j (0 .. kDmaPerWave - 1) of a tile into stage s, to constant offsets
+  // from `base`, the LDS address of the wave's first copy
+  const uint32_t lds_wave =
+      __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(lds_void*)(lds + wave * 1024));
+  auto dma = [&](uint32_t base, const rsrc_t& xr, const rsrc_t& wr, int s, int j) {
+    if (j < kXPerWave)
+      lds_dma_b128(xr, base + s * kXBytes + kWaves * j * 1024, xsrc[j]);
+    else
+      lds_dma_b128(wr, base + STAGES * kXBytes + s * kWBytes + kWaves * (j - kXPerWave) * 1024,
+                   wsrc[j - kXPerWave]);
   };
 
   // lane part of a fragment's LDS offset at k-step ks: row l32 of a 32-row
@@ -231,12 +242,16 @@ __global__ __launch_bounds__(64 * kWaves, 1) void proj_kernel(ProjParams p) {
   // the MFMAs of one k-step, with a tile's copies (into stage s) spread
   // between them when `copy` is set
   auto mma = [&](const Frags<NJ>& f, bool copy, const rsrc_t& xr, const rsrc_t& wr, int s) {
+    // (opaque, or every stage's addresses would be kept in SGPRs over the
+    // loop: 6 spilled with four stages)
+    uint32_t base = lds_wave;
+    asm volatile("" : "+s"(base));
 #pragma unroll
     for (int u = 0; u < kMfma; ++u) {
       acc[u / NJ][u % NJ] = mfma32x32x16(f.a[u / NJ], f.b[u % NJ], acc[u / NJ][u % NJ]);
       if (copy) {
 #pragma unroll
-        for (int j = u * kDmaPerWave / kMfma; j < (u + 1) * kDmaPerWave / kMfma; ++j) dma(xr, wr, s, j);
+        for (int j = u * kDmaPerWave / kMfma; j < (u + 1) * kDmaPerWave / kMfma; ++j) dma(base, xr, wr, s, j);
       }
     }
   };
@@ -249,31 +264,24 @@ __global__ __launch_bounds__(64 * kWaves, 1) void proj_kernel(ProjParams p) {
     wreg = o.norm_w_f32 ? ((const float*)o.norm_w)[tid] : bf16_bits_to_f32(((const uint16_t*)o.norm_w)[tid]);
 
   const int nt = p.K / kKTile;
-  // prologue: tiles 0 and 1 in flight, tile 0 published
-  {
-    const rsrc_t x0 = x_rsrc(0, true), w0 = w_rsrc(0, true);
+  // prologue: the first STAGES tiles in flight, tile 0 published
 #pragma unroll
-    for (int j = 0; j < kDmaPerWave; ++j) dma(x0, w0, 0, j);
-    const rsrc_t x1 = x_rsrc(1, nt > 1), w1 = w_rsrc(1, nt > 1);
+  for (int t = 0; t < STAGES; ++t) {
+    const rsrc_t xr = x_rsrc(t, t < nt), wr = w_rsrc(t, t < nt);
 #pragma unroll
-    for (int j = 0; j < kDmaPerWave; ++j) dma(x1, w1, 1, j);
-    // this wave's copies of tile 0 (tile 1's may stay in flight)
-    if constexpr (kDmaPerWave == 8) {
-      asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
-    } else {
-      static_assert(kDmaPerWave == 6, "prologue wait");
-      asm volatile("s_waitcnt vmcnt(6)" ::: "memory");
-    }
+    for (int j = 0; j < kDmaPerWave; ++j) dma(lds_wave, xr, wr, t, j);
   }
+  // this wave's copies of tile 0 (the later tiles' may stay in flight)
+  wait_lds_loads_but<(STAGES - 1) * kDmaPerWave>();
   __syncthreads();
   Frags<NJ> f0 = load(0, 0), f1;
 
   // tile t in stage S (a compile-time constant: the loop is unrolled over the
-  // two stages).  After the last tile the fragment reads of "tile t + 1"
-  // read a stale stage and the copies of "tile t + 2" are empty: both stay in
-  // bounds, their results are never used, and the loop has no branches.
+  // stages).  After the last tile the fragment reads of "tile t + 1" read a
+  // stale stage and the copies of "tile t + STAGES" are empty: both stay in
+  // bounds and their results are never used.
   auto tile = [&](auto SC, int t) {
-    constexpr int S = decltype(SC)::value, S1 = S ^ 1;
+    constexpr int S = decltype(SC)::value, S1 = (S + 1) % STAGES;
     f1 = load(S, 1);
     sched_fence();
     mma(f0, false, {}, {}, S);
@@ -287,21 +295,27 @@ __global__ __launch_bounds__(64 * kWaves, 1) void proj_kernel(ProjParams p) {
     mma(f0, false, {}, {}, S);
     sched_fence();
     // every wave has its last fragments of tile t (the barrier waits for
-    // their reads), and tile t + 1 is complete: its copies were issued in the
-    // last k-step of tile t - 1
-    wait_lds_loads();
+    // their reads), and tile t + 1 is complete: only the copies of tiles
+    // t + 2 .. t + STAGES - 1 were issued after its own
+    wait_lds_loads_but<(STAGES - 2) * kDmaPerWave>();
     __syncthreads();
-    const bool more2 = t + 2 < nt;
-    const rsrc_t xr = x_rsrc(t + 2, more2), wr = w_rsrc(t + 2, more2);
+    const bool more = t + STAGES < nt;
+    const rsrc_t xr = x_rsrc(t + STAGES, more), wr = w_rsrc(t + STAGES, more);
     f0 = load(S1, 0);
     sched_fence();
-    mma(f1, true, xr, wr, S);  // tile t + 2 into tile t's stage
+    mma(f1, true, xr, wr, S);  // tile t + STAGES into tile t's stage
     sched_fence();
   };
 #pragma unroll 1
-  for (int t = 0; t < nt; t += kStages) {
+  for (int t = 0; t < nt; t += STAGES) {
     tile(Int<0>{}, t);
     if (t + 1 < nt) tile(Int<1>{}, t + 1);
+    if constexpr (STAGES > 2) {
+      if (t + 2 < nt) tile(Int<2>{}, t + 2);
+    }
+    if constexpr (STAGES > 3) {
+      if (t + 3 < nt) tile(Int<3>{}, t + 3);
+    }
   }
   // the last tiles issued (empty) copies; none may still write the LDS when
   // the workgroup ends
@@ -312,7 +326,7 @@ __global__ __launch_bounds__(64 * kWaves, 1) void proj_kernel(ProjParams p) {
 
   // ---- epilogue: this lane holds tokens m0 + TPW tg + 32 j + l32 and
   // features 32 i + c_row(r, g) of head h, i in 0..3, j < NJ
-  const int h = hp * kBlockHeads + hh;
+  const int h = h0 + hh;
   if (h >= p.heads) return;
   const int lane_e = harp_ra::lane_id_fresh(), l32e = lane_e & 31, ge = lane_e >> 5;
 #pragma unroll
@@ -434,28 +448,59 @@ int device_cus() {
   }
   return cached[dev];
 }
+
+// One grid over all outputs, every block TPW * 4 tokens x HEADS heads.
+template <int TPW, int HEADS, int STAGES>
+hipError_t launch_grid(ProjParams p, hipStream_t stream) {
+  constexpr int kTok = kTokenGroups * TPW;
+  p.n_lin = ((p.M + kTok - 1) / kTok) * ((p.heads + HEADS - 1) / HEADS);
+  p.keep_last = p.tail_bid0 = p.n_lin;
+  hipLaunchKernelGGL((proj_kernel<TPW, HEADS, STAGES, false>), dim3((unsigned)p.n_lin, (unsigned)p.n_outs),
+                     dim3(64 * kTokenGroups * HEADS), 0, stream, p);
+  return hipGetLastError();
+}
+
+// Parts of the last r units of the 256-token x 2-head grid, as blocks of 128
+// tokens x HEADS heads.
+template <int HEADS, int STAGES>
+hipError_t launch_tail(const ProjParams& p, int r, hipStream_t stream) {
+  hipLaunchKernelGGL((proj_kernel<32, HEADS, STAGES, true>), dim3((unsigned)(4 / HEADS * r)),
+                     dim3(64 * kTokenGroups * HEADS), 0, stream, p);
+  return hipGetLastError();
+}
+
 }  // namespace
 
+// Which blocks.  Each kind is taken where one round of it covers the whole
+// grid, the smallest first: a round of the 128-token x 1-head blocks takes
+// 27-35 us at K = 3072 and 3840 (256 tokens), one of 128 x 2 heads 42-59 us
+// (300-768 tokens), one of 256 x 2 heads 70-102 us.  In two rounds the smaller
+// blocks lose: 900 tokens x 24 heads takes 72 us in large blocks and 78-81 in
+// the others, 300 tokens x 30 heads 48 us in 128 x 2 and 61 in 128 x 1.
+// Beyond one round of the large blocks, the units left over for the last one
+// run in a second launch as parts, when one round holds all of them: four
+// parts of 1 head up to a quarter of the CUs, two of 2 heads up to half (at
+// most half full, the last round would idle half the CUs through a whole
+// block).  Against a whole round: 2048 tokens x 24 heads (32 units over) 142
+// -> 116 us, 2048 x 30 (104 over) 181 -> 159.
 hipError_t launch_proj(const ProjParams& p_in, hipStream_t stream) {
   ProjParams p = p_in;
-  const int n_mt = (p.M + kBlockTokens - 1) / kBlockTokens;
-  const int n_hp = (p.heads + kBlockHeads - 1) / kBlockHeads;
-  const int L = n_mt * n_hp;
-  p.n_lin = L;
-  p.keep_last = L;
-  p.tail_bid0 = L;
-  // units left over for the last round of the CUs: when they fill at most
-  // half of it, run them as 128-token halves in a second launch
-  const int cus = device_cus();
+  const int64_t cus = device_cus();
+  const int64_t tiles128 = (int64_t)p.n_outs * ((p.M + 127) / 128);
+  if (tiles128 * p.heads <= cus) return launch_grid<32, 1, 4>(p, stream);
+  if (tiles128 * ((p.heads + 1) / 2) <= cus) return launch_grid<32, 2, 3>(p, stream);
+  const int L = ((p.M + kBlockTokens - 1) / kBlockTokens) * ((p.heads + kBlockHeads - 1) / kBlockHeads);
   const int64_t units = (int64_t)p.n_outs * L;
   const int r = cus > 0 ? (int)(units % cus) : 0;
   const bool split = r > 0 && 2 * r <= cus && units > cus && r <= L;
-  if (split) p.keep_last = p.tail_bid0 = L - r;
-  hipLaunchKernelGGL(proj_kernel<64>, dim3((unsigned)L, (unsigned)p.n_outs), dim3(64 * kWaves), 0, stream, p);
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess || !split) return e;
-  hipLaunchKernelGGL(proj_kernel<32>, dim3((unsigned)(2 * r)), dim3(64 * kWaves), 0, stream, p);
-  return hipGetLastError();
+  if (!split) return launch_grid<64, 2, 2>(p, stream);
+  p.n_lin = L;
+  p.keep_last = p.tail_bid0 = L - r;
+  hipLaunchKernelGGL((proj_kernel<64, 2, 2, false>), dim3((unsigned)L, (unsigned)p.n_outs),
+                     dim3(64 * kTokenGroups * 2), 0, stream, p);
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return e;
+  return 4 * r <= cus ? launch_tail<1, 4>(p, r, stream) : launch_tail<2, 3>(p, r, stream);
 }
 
 }  // namespace harp_proj

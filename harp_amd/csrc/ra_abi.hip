@@ -242,6 +242,13 @@ KvPlan kv_plan(double us_per_key, int batch, int h_num, int t_num, int h_len, co
   return best;
 }
 
+// Whole ring steps over as many blocks as the CUs hold: the plan of calls
+// whose workspace does not hold kv_plan's partials (take_layout).
+KvPlan ring_plan(int batch, int h_num, int t_num, const Geometry& g) {
+  const int fill = grid_fill((int64_t)((t_num + kQueryBlockRows - 1) / kQueryBlockRows) * h_num * batch);
+  return KvPlan{fill < g.n ? fill : g.n, 1, 0};
+}
+
 // The forward's and dQ's chunk table: the chunks in ring order, each as its
 // plan's pieces (a piece past a chunk's valid keys is empty).
 void fill_kv_table(ChunkTable* ct, const KvPlan& kp, const Geometry& g, const void* const* k_chunks,
@@ -291,8 +298,8 @@ struct FwdLayout {
   KvPlan kv;
   size_t o, m, l, bytes;  // byte offsets
 };
-FwdLayout fwd_layout(int batch, int h_num, int t_num, int h_len, const Geometry& g) {
-  FwdLayout w{kv_plan(kFwdUsPerKey, batch, h_num, t_num, h_len, g), 0, 0, 0, 0};
+FwdLayout fwd_layout(const KvPlan& kv, int batch, int h_num, int t_num, int h_len) {
+  FwdLayout w{kv, 0, 0, 0, 0};
   if (w.kv.n_split < 2) return w;
   const size_t rows = (size_t)batch * h_num * t_num;
   w.m = round256(sizeof(float) * w.kv.n_split * rows * h_len);
@@ -301,7 +308,7 @@ FwdLayout fwd_layout(int batch, int h_num, int t_num, int h_len, const Geometry&
   return w;
 }
 size_t fwd_ws(int batch, int h_num, int t_num, int h_len, const Geometry& g) {
-  return fwd_layout(batch, h_num, t_num, h_len, g).bytes;
+  return fwd_layout(kv_plan(kFwdUsPerKey, batch, h_num, t_num, h_len, g), batch, h_num, t_num, h_len).bytes;
 }
 
 // Backward: the per-query statistics, written once per call by the dQ
@@ -314,8 +321,9 @@ struct BwdLayout {
   QPlan q;
   size_t stats, dq, dk, dv, bytes;  // byte offsets
 };
-BwdLayout bwd_layout(int batch, int h_num, int t_num, int h_len, int kv_chunk_len, const Geometry& g) {
-  BwdLayout w{kv_plan(kDqUsPerKey, batch, h_num, t_num, h_len, g), q_plan(batch, h_num, t_num, h_len, kv_chunk_len, g.n), 0, 0, 0, 0, 0};
+BwdLayout bwd_layout(const KvPlan& kv, const QPlan& q, int batch, int h_num, int t_num, int h_len, int kv_chunk_len,
+                     const Geometry& g) {
+  BwdLayout w{kv, q, 0, 0, 0, 0, 0};
   const size_t rows = (size_t)batch * h_num * t_num, keys = (size_t)batch * h_num * g.n * kv_chunk_len;
   w.dq = w.dk = w.dv = w.bytes = round256(2 * sizeof(float) * rows);
   if (w.kv.n_split > 1) w.bytes = w.dq + round256(sizeof(float) * w.kv.n_split * rows * h_len);
@@ -327,7 +335,19 @@ BwdLayout bwd_layout(int batch, int h_num, int t_num, int h_len, int kv_chunk_le
   return w;
 }
 size_t bwd_ws(int batch, int h_num, int t_num, int h_len, int kv_chunk_len, const Geometry& g) {
-  return bwd_layout(batch, h_num, t_num, h_len, kv_chunk_len, g).bytes;
+  return bwd_layout(kv_plan(kDqUsPerKey, batch, h_num, t_num, h_len, g),
+                    q_plan(batch, h_num, t_num, h_len, kv_chunk_len, g.n), batch, h_num, t_num, h_len, kv_chunk_len, g)
+      .bytes;
+}
+
+// The layout a call runs with: the measured plan's where the caller's
+// workspace holds it, else the ring steps' alone.  So a caller that sized its
+// workspace for whole ring steps keeps it, and a call without one (a forward
+// of one chunk, say, on several streams or under capture) takes nothing from
+// the library's shared buffer that whole ring steps would not.
+template <class Layout>
+const Layout& take_layout(const Layout& planned, const Layout& ring, const void* ws, size_t ws_bytes) {
+  return planned.bytes <= (ws ? ws_bytes : ring.bytes) ? planned : ring;
 }
 
 // Library-owned grow-only workspace, one per device (used when the caller
@@ -451,7 +471,10 @@ int forward_impl(const void* q, const int64_t* q_strides, const void* const* k_c
   if (!m_i || !l_i) return fail(HARP_RA_EINVAL, "m_i / l_i are NULL");
   if (m_i_dtype != HARP_RA_F32 && m_i_dtype != HARP_RA_BF16) return fail(HARP_RA_EINVAL, "m_i_dtype must be F32 or BF16");
 
-  const FwdLayout wl = fwd_layout(batch, h_num, t_num, h_len, g);
+  const FwdLayout wl =
+      take_layout(fwd_layout(kv_plan(kFwdUsPerKey, batch, h_num, t_num, h_len, g), batch, h_num, t_num, h_len),
+                  fwd_layout(ring_plan(batch, h_num, t_num, g), batch, h_num, t_num, h_len), workspace,
+                  workspace_bytes);
   if ((rc = resolve_workspace(&workspace, &workspace_bytes, wl.bytes))) return rc;
   hipStream_t st = static_cast<hipStream_t>(stream);
 
@@ -587,7 +610,12 @@ int backward_impl(const void* q, const int64_t* q_strides, void* grad_q, const i
   if (!delta && (rc = check_plain_view(out, out_strides, "out"))) return rc;
   if (m_i_dtype != HARP_RA_F32 && m_i_dtype != HARP_RA_BF16) return fail(HARP_RA_EINVAL, "m_i_dtype must be F32 or BF16");
 
-  const BwdLayout wl = bwd_layout(batch, h_num, t_num, h_len, kv_chunk_len, g);
+  const KvPlan kv = kv_plan(kDqUsPerKey, batch, h_num, t_num, h_len, g);
+  const QPlan qp = q_plan(batch, h_num, t_num, h_len, kv_chunk_len, g.n), whole{1, (t_num + 63) / 64 * 64};
+  const BwdLayout wl = take_layout(
+      bwd_layout(kv, qp, batch, h_num, t_num, h_len, kv_chunk_len, g),
+      bwd_layout(ring_plan(batch, h_num, t_num, g), whole, batch, h_num, t_num, h_len, kv_chunk_len, g), workspace,
+      workspace_bytes);
   if ((rc = resolve_workspace(&workspace, &workspace_bytes, wl.bytes))) return rc;
   hipStream_t st = static_cast<hipStream_t>(stream);
 

@@ -171,9 +171,12 @@ HARP_RA_API int harp_ra_delta(const void* grad_out, const int64_t* do_strides,
  * needs n * B*H*T * (4*h_len + 8) bytes for the splits' partial O, m and l
  * (n <= 16), and the backward the larger of n * B*H*T * 4*h_len for the dQ
  * partials and n * B*H*sp_size*kv_chunk_len * 8*h_len (n <= 8) for the dK and
- * dV partials (each part rounded up to 256 bytes).  Replaces the reference's grow-only scratch sizing
- * (RingAttnHbmWorkspace::ensure_slot, ring_attn.cpp:620-840, sized at
- * :2428-2450 and :2595-2656).
+ * dV partials (each part rounded up to 256 bytes).  A call with a smaller
+ * workspace, or none, splits at most whole ring steps, over up to sp_size
+ * blocks (n <= sp_size for the forward and dQ, dK / dV whole); a workspace too
+ * small for that is refused with HARP_RA_ENOMEM.  Replaces the reference's
+ * grow-only scratch sizing (RingAttnHbmWorkspace::ensure_slot,
+ * ring_attn.cpp:620-840, sized at :2428-2450 and :2595-2656).
  */
 HARP_RA_API size_t harp_ra_forward_workspace_bytes(int batch, int h_num, int t_num, int h_len, int sp_size,
                                        int kv_chunk_len, const int32_t* kv_valid_lens);

@@ -70,15 +70,35 @@ def test_split_calls_against_fp64(B, H, T, D, sp, chunk, lens, rank, grads):
     assert not dk[:, :, ~keep].any() and not dv[:, :, ~keep].any()
 
 
-def test_a_smaller_workspace_is_refused():
+def test_a_smaller_workspace_keeps_whole_grids():
+    """A workspace for the statistics alone (all that whole grids need) is
+    taken; a smaller one is refused."""
     lib = harp_amd.load_abi()
-    need = H_ops.backward_workspace_bytes(1, 2, 1024, 128, 1, 1024)
-    assert need > 2 * 4 * 2 * 1024  # more than the statistics: split partials
+    B, H, T, D = 1, 2, 1024, 128
+    need, stats = H_ops.backward_workspace_bytes(B, H, T, D, 1, T), 2 * 4 * H * T
+    assert need > stats  # split partials
+    assert H_ops.forward_workspace_bytes(B, H, T, D, 1, T) > 0
     g = torch.Generator(device=DEV).manual_seed(1)
-    q = torch.randn(1, 1024, 2, 128, device=DEV, generator=g).to(torch.bfloat16).transpose(1, 2)
-    f = torch.zeros(1, 2, 1024, device=DEV)
-    ws = torch.empty(need - 256, dtype=torch.uint8, device=DEV)
+    q, k, v, dout = (torch.randn(B, T, H, D, device=DEV, generator=g).to(torch.bfloat16).transpose(1, 2) for _ in range(4))
+    o64, dq64, dk64, dv64, _ = _ref(q, k, v, dout, torch.ones(T, dtype=torch.bool, device=DEV))
+    out, delta = torch.empty_like(q, dtype=torch.float32), torch.empty(B, H, T, device=DEV)
+    m, l = torch.empty_like(delta), torch.empty_like(delta)
+    scale = 1.0 / math.sqrt(D)
+    none = torch.empty(0, dtype=torch.uint8, device=DEV)  # a NULL workspace
+    H_ops.abi_forward(q, [k], [v], out, m, l, scale, workspace=none)
+    H_ops.abi_delta(dout, out, delta)
+    grads = [torch.empty_like(q) for _ in range(3)]
+
+    def backward(nbytes):
+        ws = torch.empty(nbytes, dtype=torch.uint8, device=DEV)
+        H_ops.abi_backward(q, grads[0], [k], [v], [grads[1]], [grads[2]], dout, m, l, delta, scale, workspace=ws)
+
+    for nbytes in (stats, need - 256, need):
+        for t in grads:
+            t.fill_(float("nan"))
+        backward(nbytes)
+        for name, a, b in (("o", out, o64), ("dq", grads[0], dq64), ("dk", grads[1], dk64), ("dv", grads[2], dv64)):
+            assert _rel(a, b) <= 3 * 2.0 ** -9, (name, nbytes, _rel(a, b))
     with pytest.raises(RuntimeError, match="workspace"):
-        H_ops.abi_backward(q, torch.empty_like(q), [q], [q], [torch.empty_like(q)], [torch.empty_like(q)], q, f, f, f,
-                           1.0, workspace=ws)
+        backward(stats - 256)
     assert "smaller" in lib.harp_ra_last_error().decode()

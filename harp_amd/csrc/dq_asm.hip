@@ -91,7 +91,9 @@ __global__ __launch_bounds__(64 * kAsmWaves, 1) void dq_asm_kernel(BwdParams p) 
     // dO's are read back from LDS, so the block pays no launch and no second
     // read of dO for it (delta_kernel took 4 us at 30 heads x 256 rows, 24 us
     // at 24 x 8192).  One forward + backward at 30 x 256 rows, 8 chunks: 128
-    // us before, 102 with D, the cast and the fill of m in these kernels
+    // us before, 102 with D, the cast and the fill of m in these kernels.
+    // The sums run in delta_kernel's order (8 elements of a lane in turn, then
+    // lanes 8, 4, 2, 1 apart), so both entry points give the same D and dS
     const int sub = lane & 15, rr = lane >> 4;
     f32x4u ox[16], oy[16];
     if (!p.delta) {
@@ -113,10 +115,7 @@ __global__ __launch_bounds__(64 * kAsmWaves, 1) void dq_asm_kernel(BwdParams p) 
         const bf16x8 x = *(const bf16x8*)(lds + 65536 + row * 256 + ((sub ^ swz(row)) << 4));
         float acc = 0.f;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          acc = __builtin_fmaf((float)x[j], ox[i][j], acc);
-          acc = __builtin_fmaf((float)x[j + 4], oy[i][j], acc);
-        }
+        for (int j = 0; j < 8; ++j) acc = __builtin_fmaf((float)x[j], j < 4 ? ox[i][j] : oy[i][j - 4], acc);
         dsum[i] = acc;
       }
       // 16 sums over the 16 lanes of a row at once: each exchange halves the

@@ -649,7 +649,8 @@ __global__ __launch_bounds__(64 * kFwdWaves, 1) void fwd_kernel(FwdParams p) {
 }
 
 // ---------------------------------------------------------------------------
-// D = rowsum(dO * O): 16 lanes per row, 8 elements per lane
+// D = rowsum(dO * O): 16 lanes per row, 8 elements per lane (the dQ kernels
+// sum in the same order where they form D themselves)
 // ---------------------------------------------------------------------------
 __global__ __launch_bounds__(256) void delta_kernel(DeltaParams p) {
   const int64_t row = (int64_t)blockIdx.x * 16 + (threadIdx.x >> 4);
@@ -665,7 +666,7 @@ __global__ __launch_bounds__(256) void delta_kernel(DeltaParams p) {
       const bf16x8 g8 = *(const bf16x8*)(p.dout + (int64_t)b * p.sdb + (int64_t)h * p.sdh + (int64_t)t * p.sdt + d0);
       const float* orow = p.out + (int64_t)b * p.sob + (int64_t)h * p.soh + (int64_t)t * p.sot + d0;
 #pragma unroll
-      for (int j = 0; j < 8; ++j) acc += (float)g8[j] * orow[j];
+      for (int j = 0; j < 8; ++j) acc = __builtin_fmaf((float)g8[j], orow[j], acc);
     }
   }
 #pragma unroll
@@ -754,22 +755,27 @@ __global__ __launch_bounds__(64 * kDqWaves, 1) void dq_kernel(BwdParams p) {
     if (q_ok) st1 = -p.delta[si];
   } else {
     // D = rowsum(dO O) here, from the dO fragments the lane holds anyway (its
-    // two lane halves each cover half of the row): no launch for it
-    float acc = 0.f;
+    // two lane halves hold the even and the odd 8-element chunks of the row):
+    // no launch for it.  Summed in delta_kernel's order, the chunks' own sums
+    // 8, 4, 2 and (between the halves) 1 chunks apart, so both entry points
+    // give the same D and dS
+    float cs[8];
     const float* orow = p.out + (int64_t)b * p.sob + (int64_t)h * p.soh + (int64_t)qi * p.sot;
 #pragma unroll
-    for (int ks = 0; ks < KSTEPS; ++ks) {
+    for (int ks = 0; ks < 8; ++ks) {
+      cs[ks] = 0.f;
       const int d0 = ks * 16 + g * 8;
-      if (q_ok && d0 < p.D) {
+      if (ks < KSTEPS && q_ok && d0 < p.D) {
         const f32x4u x = *(const f32x4u*)(orow + d0), y = *(const f32x4u*)(orow + d0 + 4);
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          acc = __builtin_fmaf((float)gf[ks][j], x[j], acc);
-          acc = __builtin_fmaf((float)gf[ks][j + 4], y[j], acc);
-        }
+        for (int j = 0; j < 8; ++j) cs[ks] = __builtin_fmaf((float)gf[ks < KSTEPS ? ks : 0][j], j < 4 ? x[j] : y[j - 4], cs[ks]);
       }
     }
-    st1 = -wave_half_sum(acc);
+#pragma unroll
+    for (int w = 4; w >= 1; w >>= 1)
+#pragma unroll
+      for (int ks = 0; ks < w; ++ks) cs[ks] += cs[ks + w];
+    st1 = -wave_half_sum(cs[0]);
   }
   if (q_ok && g == 0 && sp.index == 0) {
     p.stats[si] = st0;

@@ -60,7 +60,8 @@ __device__ __forceinline__ float dpp(float v) {
   return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), CTRL, 0xf, 0xf, true));
 }
 // sum over the LPR lanes of a group, the same in every lane (each step adds
-// the same two values in both partners)
+// the same two values in both partners): lanes 8 (16 per row), 4, 2 and 1
+// apart, so a row's sum is the same fp32 value with 8 and with 16 lanes
 template <int LPR>
 __device__ __forceinline__ float group_sum(float v) {
   static_assert(LPR == 16 || LPR == 8);
@@ -68,7 +69,7 @@ __device__ __forceinline__ float group_sum(float v) {
     v += dpp<0x128>(v);  // row_ror:8
     v += dpp<0x124>(v);  // row_ror:4
   } else {
-    v += dpp<0x141>(v);  // row_half_mirror
+    v += dpp<0x1b>(dpp<0x141>(v));  // row_half_mirror, then quad_perm:[3,2,1,0]: lane ^ 4
   }
   v += dpp<0x4e>(v);  // quad_perm:[2,3,0,1]
   v += dpp<0xb1>(v);  // quad_perm:[1,0,3,2]

@@ -65,3 +65,26 @@ def test_large_call_equals_small_calls(op, D, layout):
     # fp32 sums of B*H*S terms, plus (norm_rope) single bf16 units of 2^-8
     # where fp64 and fp32 truncate apart: a few in 1e5 elements
     assert float((gw.double() - ref).norm() / ref.norm()) <= 1e-4
+
+
+@pytest.mark.parametrize("D", [8, 24, 32, 40, 56, 64])
+def test_row_sums_do_not_depend_on_the_lanes_per_row(D):
+    """Rows of up to 64 elements (8 lanes each) against the same rows padded
+    with zeros to four (D = 8: sixteen) times the length (16 lanes): the sum of
+    squares is one fp32 tree, its mean differs by a power of four, so rms and y
+    agree to the bit after scaling by that power's root."""
+    harp_amd.load_async_ops()
+    g = torch.Generator(device=DEV).manual_seed(D)
+    x = torch.randn(1, 3, 2000, D, device=DEV, generator=g).to(torch.bfloat16)
+    r = 4 if D == 8 else 2
+
+    def norm(x, eps):
+        y, rms = torch.empty_like(x), torch.empty(3 * 2000, device=DEV)
+        w = torch.ones(x.size(-1), dtype=torch.bfloat16, device=DEV)
+        torch.ops.async_op.rmsnorm_forward_out(x, w, y, rms, eps)
+        return y, rms
+
+    y, rms = norm(x, 2.0 ** -16)
+    ypad, rpad = norm(torch.nn.functional.pad(x, (0, D * (r * r - 1))), 2.0 ** -16 / r ** 2)
+    assert torch.equal(rms, rpad * r)
+    assert torch.equal(y * r, ypad[..., :D])

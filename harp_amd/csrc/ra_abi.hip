@@ -243,7 +243,8 @@ KvPlan kv_plan(double us_per_key, int batch, int h_num, int t_num, int h_len, co
 }
 
 // Whole ring steps over as many blocks as the CUs hold: the plan of calls
-// whose workspace does not hold kv_plan's partials (take_layout).
+// whose workspace does not hold kv_plan's partials (take_layout).  One chunk
+// has no ring steps to split: the forward then needs no workspace.
 KvPlan ring_plan(int batch, int h_num, int t_num, const Geometry& g) {
   const int fill = grid_fill((int64_t)((t_num + kQueryBlockRows - 1) / kQueryBlockRows) * h_num * batch);
   return KvPlan{fill < g.n ? fill : g.n, 1, 0};
@@ -342,9 +343,8 @@ size_t bwd_ws(int batch, int h_num, int t_num, int h_len, int kv_chunk_len, cons
 
 // The layout a call runs with: the measured plan's where the caller's
 // workspace holds it, else the ring steps' alone.  So a caller that sized its
-// workspace for whole ring steps keeps it, and a call without one (a forward
-// of one chunk, say, on several streams or under capture) takes nothing from
-// the library's shared buffer that whole ring steps would not.
+// workspace for whole ring steps keeps it, and a call without one takes
+// nothing from the library's shared buffer that whole ring steps would not.
 template <class Layout>
 const Layout& take_layout(const Layout& planned, const Layout& ring, const void* ws, size_t ws_bytes) {
   return planned.bytes <= (ws ? ws_bytes : ring.bytes) ? planned : ring;
@@ -471,10 +471,14 @@ int forward_impl(const void* q, const int64_t* q_strides, const void* const* k_c
   if (!m_i || !l_i) return fail(HARP_RA_EINVAL, "m_i / l_i are NULL");
   if (m_i_dtype != HARP_RA_F32 && m_i_dtype != HARP_RA_BF16) return fail(HARP_RA_EINVAL, "m_i_dtype must be F32 or BF16");
 
+  // harp_ra_forward of one chunk needs no workspace and so leaves alone what it
+  // is given (calls on several streams may share it, at any alignment): its
+  // keys are split only by harp_ra_forward_rounded
+  const FwdLayout ring = fwd_layout(ring_plan(batch, h_num, t_num, g), batch, h_num, t_num, h_len);
+  const FwdLayout planned =
+      fwd_layout(kv_plan(kFwdUsPerKey, batch, h_num, t_num, h_len, g), batch, h_num, t_num, h_len);
   const FwdLayout wl =
-      take_layout(fwd_layout(kv_plan(kFwdUsPerKey, batch, h_num, t_num, h_len, g), batch, h_num, t_num, h_len),
-                  fwd_layout(ring_plan(batch, h_num, t_num, g), batch, h_num, t_num, h_len), workspace,
-                  workspace_bytes);
+      !out_rounded && ring.bytes == 0 ? ring : take_layout(planned, ring, workspace, workspace_bytes);
   if ((rc = resolve_workspace(&workspace, &workspace_bytes, wl.bytes))) return rc;
   hipStream_t st = static_cast<hipStream_t>(stream);
 

@@ -178,7 +178,7 @@ std::tuple<at::Tensor, at::Tensor, at::Tensor> forward_hip(const at::Tensor& q, 
   const int32_t* lens = ch.lens.empty() ? nullptr : ch.lens.data();
   const size_t ws_bytes = harp_ra_forward_workspace_bytes(B, H, T, D, sp_size, ch.chunk_len, lens);
   check_status(ws_bytes != SIZE_MAX ? HARP_RA_OK : HARP_RA_EINVAL, "ring_attention_forward");
-  at::Tensor ws = workspace(ws_bytes, q);
+  at::Tensor ws = workspace(sp_size > 1 ? ws_bytes : 0, q);  // one chunk: harp_ra_forward takes none
   const auto qs = strides4(q), ks = strides4(k), os = strides4(out);
   hipStream_t stream = c10::hip::getCurrentHIPStream(q.get_device()).stream();
   const int rc = harp_ra_forward(q.data_ptr(), qs.data(), ch.k.data(), ch.v.data(), ks.data(), ch.chunk_len, lens,

@@ -61,9 +61,10 @@ enum { HARP_RA_F32 = 0, HARP_RA_BF16 = 1 };
  *   int t_num, int h_num, int h_len, int sp_size, __bf16* m_i, float* l_i,
  *   float scale)  — gemm/ring_attention/ring_attn.cpp:2412-2414, called from
  *   ring_attention_forward_op, torch_ring_attention_ops.cpp:177-215.
- * workspace: harp_ra_forward_workspace_bytes() bytes of device memory, or
- * NULL to use a grow-only per-device buffer owned by the library (calls with
- * a NULL workspace that overlap on one device then race).
+ * workspace: harp_ra_forward_workspace_bytes() bytes of device memory
+ * (256-byte aligned), or NULL to use a grow-only per-device buffer owned by
+ * the library (calls with a NULL workspace that overlap on one device then
+ * race).  With sp_size 1 none is needed and what is passed is left alone.
  */
 HARP_RA_API int harp_ra_forward(const void* q, const int64_t* q_strides,
                     const void* const* k_chunks, const void* const* v_chunks,
@@ -82,7 +83,9 @@ HARP_RA_API int harp_ra_forward(const void* q, const int64_t* q_strides,
  * read 4 bytes and write 2 per element for.  out_rounded is a [B,H,T,D] view
  * as out, its pointer 8-byte aligned and its strides (of dims longer than 1)
  * multiples of 4 elements; out may be NULL (its strides are then ignored) when
- * no backward follows.  Everything else as harp_ra_forward.
+ * no backward follows.  Everything else as harp_ra_forward, except that with
+ * sp_size 1 a workspace is used here too, where it holds the splits' partials
+ * (harp_ra_forward_workspace_bytes); without one the keys are not split.
  */
 HARP_RA_API int harp_ra_forward_rounded(const void* q, const int64_t* q_strides,
                     const void* const* k_chunks, const void* const* v_chunks,
@@ -174,7 +177,9 @@ HARP_RA_API int harp_ra_delta(const void* grad_out, const int64_t* do_strides,
  * dV partials (each part rounded up to 256 bytes).  A call with a smaller
  * workspace, or none, splits at most whole ring steps, over up to sp_size
  * blocks (n <= sp_size for the forward and dQ, dK / dV whole); a workspace too
- * small for that is refused with HARP_RA_ENOMEM.  Replaces the reference's
+ * small for that is refused with HARP_RA_ENOMEM.  harp_ra_forward with
+ * sp_size 1 needs none whatever this returns (only harp_ra_forward_rounded
+ * uses it there).  Replaces the reference's
  * grow-only scratch sizing (RingAttnHbmWorkspace::ensure_slot,
  * ring_attn.cpp:620-840, sized at :2428-2450 and :2595-2656).
  */

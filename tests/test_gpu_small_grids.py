@@ -1,6 +1,6 @@
 """GPU: calls whose grids leave most CUs idle, where the forward and dQ split
-the keys of a chunk (not only the ring steps) and dK/dV splits the queries,
-against fp64 attention: piece edges, pad keys that leave pieces empty, several
+the keys of a chunk (not only the ring steps; harp_ra_forward of a single chunk
+stays whole) and dK/dV splits the queries, against fp64 attention: piece edges, pad keys that leave pieces empty, several
 chunks in rotated ring order, bf16 and fp32 gradients, unaligned bf16 views."""
 
 import math
@@ -102,3 +102,50 @@ def test_a_smaller_workspace_keeps_whole_grids():
     with pytest.raises(RuntimeError, match="workspace"):
         backward(stats - 256)
     assert "smaller" in lib.harp_ra_last_error().decode()
+
+
+@pytest.mark.parametrize("D", [64, 128])
+def test_forward_of_one_chunk_leaves_its_workspace_alone(D):
+    """harp_ra_forward of one chunk needs no workspace: a buffer that is passed
+    all the same is neither written nor refused for its alignment, so calls on
+    several streams may be handed the same one."""
+    B, H, T = 1, 2, 1024
+    g = torch.Generator(device=DEV).manual_seed(2)
+    q, k, v = (torch.randn(B, T, H, D, device=DEV, generator=g).to(torch.bfloat16).transpose(1, 2) for _ in range(3))
+    nbytes = H_ops.forward_workspace_bytes(B, H, T, D, 1, T)
+    assert nbytes > 0  # the size at which harp_ra_forward_rounded splits the keys
+    buf = torch.full((nbytes + 512,), 0x5a, dtype=torch.uint8, device=DEV)
+    res = []
+    for ws in (torch.empty(0, dtype=torch.uint8, device=DEV), buf, buf[8:]):
+        out, m, l = torch.empty_like(q, dtype=torch.float32), torch.empty(B, H, T, device=DEV), torch.empty(B, H, T, device=DEV)
+        H_ops.abi_forward(q, [k], [v], out, m, l, 1.0 / math.sqrt(D), workspace=ws)
+        res.append((out, m, l))
+    assert bool((buf == 0x5a).all())
+    for r in res[1:]:
+        assert all(torch.equal(a, b) for a, b in zip(r, res[0]))
+
+
+@pytest.mark.parametrize("B,H,T,D,sp,chunk,lens,rank", SHAPES)
+def test_one_call_operators_on_small_grids(B, H, T, D, sp, chunk, lens, rank):
+    """The same shapes through ring_attention_attend / ring_attention_grad,
+    which split the keys of a single chunk too: the rounded output stored by
+    the merge, D formed by each key piece's dQ block."""
+    harp_amd.load_ops()
+    ops = torch.ops.ring_attention_ops
+    g = torch.Generator(device=DEV).manual_seed(T + D)
+    q, dout = (torch.randn(B, T, H, D, device=DEV, generator=g).to(torch.bfloat16).transpose(1, 2) for _ in range(2))
+    k, v = (torch.randn(B, sp * chunk, H, D, device=DEV, generator=g).to(torch.bfloat16).transpose(1, 2) for _ in range(2))
+    pos = torch.arange(sp * chunk, device=DEV)
+    keep = (pos % chunk) < torch.tensor(lens, device=DEV)[pos // chunk]
+    o64, dq64, dk64, dv64, lse64 = _ref(q, k, v, dout, keep)
+    scale = 1.0 / math.sqrt(D)
+    o, out, m, l = ops.ring_attention_attend(q, k, v, sp, scale, rank, lens, chunk)
+    assert torch.equal(o, out.to(torch.bfloat16))
+    only, none, m1, l1 = ops.ring_attention_attend(q, k, v, sp, scale, rank, lens, chunk, False)
+    assert torch.equal(only, o) and none.numel() == 0 and torch.equal(m1, m) and torch.equal(l1, l)
+    dq, dk, dv = ops.ring_attention_grad(dout, q, k, v, out, m, l, sp, scale, rank, lens, chunk)
+    assert float(((m.double() + l.double().log()).squeeze(-1) - lse64).abs().max()) <= 1e-4
+    # as test_split_calls_against_fp64
+    for name, a, b in (("o", out, o64), ("dq", dq, dq64), ("dk", dk[:, :, keep], dk64), ("dv", dv[:, :, keep], dv64)):
+        assert _rel(a, b) <= 3 * 2.0 ** -9, (name, _rel(a, b))
+    assert not dk[:, :, ~keep].any() and not dv[:, :, ~keep].any()

@@ -342,7 +342,8 @@ size_t bwd_ws(int batch, int h_num, int t_num, int h_len, int kv_chunk_len, cons
 }
 
 // The layout a call runs with: the measured plan's where the caller's
-// workspace holds it, else the ring steps' alone.  So a caller that sized its
+// workspace holds it or, without a workspace, where it takes no more than the
+// ring steps' alone would; else the ring steps'.  So a caller that sized its
 // workspace for whole ring steps keeps it, and a call without one takes
 // nothing from the library's shared buffer that whole ring steps would not.
 template <class Layout>

@@ -174,12 +174,12 @@ HARP_RA_API int harp_ra_delta(const void* grad_out, const int64_t* do_strides,
  * needs n * B*H*T * (4*h_len + 8) bytes for the splits' partial O, m and l
  * (n <= 16), and the backward the larger of n * B*H*T * 4*h_len for the dQ
  * partials and n * B*H*sp_size*kv_chunk_len * 8*h_len (n <= 8) for the dK and
- * dV partials (each part rounded up to 256 bytes).  A call with a smaller
- * workspace, or none, splits at most whole ring steps, over up to sp_size
- * blocks (n <= sp_size for the forward and dQ, dK / dV whole); a workspace too
- * small for that is refused with HARP_RA_ENOMEM.  harp_ra_forward with
- * sp_size 1 needs none whatever this returns (only harp_ra_forward_rounded
- * uses it there).  Replaces the reference's
+ * dV partials (each part rounded up to 256 bytes).  That plan runs where the
+ * call's workspace holds it or, with none passed, where it takes no more than
+ * splitting whole ring steps would (over min(sp_size, CUs / tiles) blocks for
+ * the forward and dQ, dK / dV whole).  Any other call splits whole ring steps;
+ * a workspace that holds neither plan is refused with HARP_RA_ENOMEM.  harp_ra_forward with sp_size 1 needs none whatever this
+ * returns (only harp_ra_forward_rounded uses it there).  Replaces the reference's
  * grow-only scratch sizing (RingAttnHbmWorkspace::ensure_slot,
  * ring_attn.cpp:620-840, sized at :2428-2450 and :2595-2656).
  */

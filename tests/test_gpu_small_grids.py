@@ -104,6 +104,39 @@ def test_a_smaller_workspace_keeps_whole_grids():
     assert "smaller" in lib.harp_ra_last_error().decode()
 
 
+def test_a_plan_below_the_ring_steps_runs_without_a_workspace():
+    """Two short chunks and many queries: dK/dV splits the queries in less
+    memory than two dQ splits by ring steps would take.  That plan runs with a
+    workspace of exactly its size and, from the library's buffer, with none."""
+    B, H, T, D, chunk = 1, 8, 2048, 128, 64
+    need = H_ops.backward_workspace_bytes(B, H, T, D, 2, chunk)
+    stats, ring = 2 * 4 * B * H * T, 2 * 4 * B * H * T + 2 * 4 * B * H * T * D
+    assert stats < need < ring and (need - stats) % (B * H * 2 * chunk * 8 * D) == 0
+    g = torch.Generator(device=DEV).manual_seed(3)
+    q, dout = (torch.randn(B, T, H, D, device=DEV, generator=g).to(torch.bfloat16).transpose(1, 2) for _ in range(2))
+    k, v = (torch.randn(B, 2 * chunk, H, D, device=DEV, generator=g).to(torch.bfloat16).transpose(1, 2) for _ in range(2))
+    o64, dq64, dk64, dv64, _ = _ref(q, k, v, dout, torch.ones(2 * chunk, dtype=torch.bool, device=DEV))
+    ch = lambda t: [t[:, :, c * chunk:(c + 1) * chunk] for c in range(2)]  # noqa: E731
+    out, delta = torch.empty_like(q, dtype=torch.float32), torch.empty(B, H, T, device=DEV)
+    m, l = torch.empty_like(delta), torch.empty_like(delta)
+    scale = 1.0 / math.sqrt(D)
+    H_ops.abi_forward(q, ch(k), ch(v), out, m, l, scale)
+    H_ops.abi_delta(dout, out, delta)
+
+    def backward(nbytes):
+        grads = [torch.full_like(t, float("nan")) for t in (q, k, v)]
+        ws = torch.empty(nbytes, dtype=torch.uint8, device=DEV)
+        H_ops.abi_backward(q, grads[0], ch(k), ch(v), ch(grads[1]), ch(grads[2]), dout, m, l, delta, scale, workspace=ws)
+        return grads
+
+    for nbytes in (need, 0):  # 0: a NULL workspace
+        for name, a, b in zip(("dq", "dk", "dv"), backward(nbytes), (dq64, dk64, dv64)):
+            assert _rel(a, b) <= 3 * 2.0 ** -9, (name, nbytes, _rel(a, b))
+    assert all(torch.equal(a, b) for a, b in zip(backward(need), backward(0)))
+    with pytest.raises(RuntimeError, match="workspace"):
+        backward(need - 256)
+
+
 @pytest.mark.parametrize("D", [64, 128])
 def test_forward_of_one_chunk_leaves_its_workspace_alone(D):
     """harp_ra_forward of one chunk needs no workspace: a buffer that is passed

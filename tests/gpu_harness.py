@@ -111,3 +111,28 @@ def run_hip(
     cpu = {k: v.cpu() for k, v in res.items()}
     cpu["lse"] = cpu["m"].double() + torch.log(cpu["l"].double())
     return cpu
+
+
+def split_plan(B, H, T, D, sp, chunk, lens=None):
+    """(forward, dQ, dK/dV): the number of blocks each of a tile's keys
+    (queries, for dK/dV) is split over with a workspace of the library's own
+    size, read off those sizes: a test of a split asserts that its shape is
+    one.  dQ's part of the backward's size is what is left when dK/dV's grid is
+    full (the same valid keys in very long chunks), dK/dV's when no key is
+    valid."""
+    lens = [chunk] * sp if lens is None else list(lens)
+
+    def r256(n):
+        return (n + 255) // 256 * 256
+
+    def invert(nbytes, size):
+        return next(n for n in range(1, 17) if nbytes == (size(n) if n > 1 else 0))
+
+    rows, keys = B * H * T, B * H * sp * chunk
+    stats = r256(8 * rows)
+    dq = hops.backward_workspace_bytes(B, H, T, D, sp, 1 << 24, lens) - stats
+    dkdv = hops.backward_workspace_bytes(B, H, T, D, sp, chunk, [0] * sp) - stats
+    assert hops.backward_workspace_bytes(B, H, T, D, sp, chunk, lens) == stats + max(dq, dkdv)
+    return (invert(hops.forward_workspace_bytes(B, H, T, D, sp, chunk, lens),
+                   lambda n: r256(4 * n * rows * D) + 2 * r256(4 * n * rows)),
+            invert(dq, lambda n: r256(4 * n * rows * D)), invert(dkdv, lambda n: 2 * r256(4 * n * keys * D)))

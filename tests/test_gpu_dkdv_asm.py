@@ -15,7 +15,7 @@ import pytest
 import torch
 
 from oracle import ring_attn_oracle as orc
-from tests.gpu_harness import run_hip
+from tests.gpu_harness import run_hip, split_plan
 from tests.parity import TOL_GRAD, rel_fro
 from tests.test_gpu_parity import _check_all, _oracle_full
 
@@ -120,7 +120,7 @@ def test_unaligned_dk_dv_views_compiled_kernel(grad_dtype, head_dim):
     _views_match(head_dim, (1, 1), grad_dtype, seed=34)
 
 
-@pytest.mark.parametrize("heads", [3, 72])  # 6 query tiles: KV split and merge; 144: the kernel's own stores
+@pytest.mark.parametrize("heads", [3, 72])  # 6 query tiles: keys split, dq_merge_kernel's stores; 144: the dQ kernel's own
 @pytest.mark.parametrize("head_dim,view", [(64, (1, 1)), (72, (3, 1)), (128, (4, 0))])
 @pytest.mark.parametrize("grad_dtype", [torch.bfloat16, torch.float32])
 def test_strided_dq_views(head_dim, view, grad_dtype, heads):
@@ -130,11 +130,28 @@ def test_strided_dq_views(head_dim, view, grad_dtype, heads):
     per lane), at 128 with padded, 8-byte aligned rows (the C ABI refuses
     other bf16 dQ views there)."""
     print(f"[dq strided views D={head_dim} {view} {grad_dtype} H={heads}]", flush=True)
-    q, ks, vs, do = orc.make_inputs(1, heads, 300, head_dim, 2, seed=35, chunk_len=200)
+    assert (split_plan(1, heads, 300, head_dim, 2, 600)[1] > 1) == (heads == 3)
+    q, ks, vs, do = orc.make_inputs(1, heads, 300, head_dim, 2, seed=35, chunk_len=600)
     scale = 1.0 / math.sqrt(head_dim)
     res = run_hip(q, ks, vs, do, scale, grad_dtype=grad_dtype)
     got = run_hip(q, ks, vs, do, scale, grad_dtype=grad_dtype, dq_view=view)
     assert torch.equal(res["dq"], got["dq"])
+
+
+@pytest.mark.parametrize("head_dim,view", [(64, (1, 1)), (72, (3, 1)), (128, (4, 0))])
+@pytest.mark.parametrize("grad_dtype", [torch.bfloat16, torch.float32])
+def test_strided_dk_dv_views_of_split_queries(head_dim, view, grad_dtype):
+    """dK / dV merged into strided views equal the plain call's bit for bit
+    (dkdv_merge_kernel's wide and element stores), pad keys included."""
+    lens = [130, 90]
+    assert split_plan(1, 2, 1500, head_dim, 2, 130, lens)[2] > 1
+    q, ks, vs, do = orc.make_inputs(1, 2, 1500, head_dim, 2, seed=36, chunk_len=130)
+    scale = 1.0 / math.sqrt(head_dim)
+    res = run_hip(q, ks, vs, do, scale, kv_lens=lens, grad_dtype=grad_dtype)
+    got = run_hip(q, ks, vs, do, scale, kv_lens=lens, grad_dtype=grad_dtype, dkv_view=view)
+    for name in ("dk", "dv"):
+        assert torch.equal(res[name], got[name]), name
+    assert torch.count_nonzero(got["dk"][:, :, 130 + 90:]) == 0
 
 
 @pytest.mark.skip(reason="head dim 128 stores bf16 dK / dV 8 bytes per lane: the C ABI refuses chunks that are not "

@@ -14,7 +14,7 @@ import pytest
 import torch
 
 from oracle import ring_attn_oracle as orc
-from tests.gpu_harness import run_hip
+from tests.gpu_harness import run_hip, split_plan
 from tests.parity import TOL_GRAD, rel_fro
 from tests.test_gpu_parity import _check_all, _oracle_full
 
@@ -65,6 +65,7 @@ def test_kv_split_small_grid():
     ring over grid dimension y; each split writes its own dQ partial."""
     q, ks, vs, do = orc.make_inputs(1, 1, 256, D, 8, seed=91, chunk_len=160)
     lens = [160, 131, 160, 7, 160, 160, 96, 160]
+    assert split_plan(1, 1, 256, D, 8, 160, lens)[1] == 8
     scale = 1.0 / math.sqrt(D)
     res = run_hip(q, ks, vs, do, scale, ring_rank=5, kv_lens=lens)
     ref = _oracle_full(q, ks, vs, do, scale, rank=5, lens=lens)

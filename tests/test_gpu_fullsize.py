@@ -12,7 +12,7 @@ import pytest
 import torch
 
 from oracle import ring_attn_oracle as orc
-from tests.gpu_harness import run_hip
+from tests.gpu_harness import run_hip, split_plan
 from tests.gpu_reference import attention_fp32
 from tests.parity import TOL_GRAD, TOL_LSE, TOL_O, rel_fro
 
@@ -76,6 +76,8 @@ def _inputs(B, H, T, D, N, tc, vscale, seed=3407):
 ])
 def test_full_size_against_fp32_reference(config, B, H, T, D, N, tc, lens, vscale):
     print(f"[config {config} full size]", flush=True)
+    kv = {"harp-256": 8, "harp-768": 2}.get(config, 1)
+    assert split_plan(B, H, T, D, N, tc, lens) == (kv, kv, 1)
     q, ks, vs, do = _inputs(B, H, T, D, N, tc, vscale)
     scale = 1.0 / math.sqrt(D)
     res = run_hip(q.cpu(), [k.cpu() for k in ks], [v.cpu() for v in vs], do.cpu(), scale, kv_lens=lens,

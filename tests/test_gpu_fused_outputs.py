@@ -9,13 +9,15 @@ import pytest
 import torch
 
 import harp_amd
+from tests.gpu_harness import split_plan
 
 pytestmark = pytest.mark.gpu
 
 DEV = "cuda:0"
 
 # (D, B, H, T, sp, chunk, valid): staged and unstaged epilogues, one row, tile
-# edges, a split over the chunks (few tiles, sp > 1), pad keys
+# edges, a split over the chunks (3 heads, 8 chunks), pad keys; key pieces and
+# query splits: tests/test_gpu_small_grids.py
 SHAPES = [
     (64, 1, 2, 1, 1, 40, 40), (64, 2, 3, 257, 4, 130, 130), (72, 1, 2, 255, 2, 200, 190),
     (96, 1, 2, 256, 1, 128, 128), (96, 1, 2, 129, 3, 64, 50), (104, 1, 2, 33, 2, 70, 70),
@@ -36,6 +38,7 @@ def test_one_call_operators_match_the_separate_ones(D, B, H, T, sp, chunk, valid
     q, dout = _view(g, B, H, T, D), _view(g, B, H, T, D)
     k, v = _view(g, B, H, sp * chunk, D), _view(g, B, H, sp * chunk, D)
     lens = None if valid == chunk else [valid] * sp
+    assert (H, sp) != (3, 8) or split_plan(B, H, T, D, sp, chunk, lens) == (8, 8, 1)
     scale = 1.0 / math.sqrt(D)
     out = torch.empty_like(q, dtype=torch.float32)
     m = torch.empty(B, H, T, 1, device=DEV, dtype=torch.bfloat16)

@@ -1,5 +1,7 @@
 """HIP-graph capture of the block's operators: ring-attention forward, delta
-and backward (torch.ops.ring_attention_ops), the fused QK RMSNorm + RoPE
+and backward and the one-call attend and grad (torch.ops.ring_attention_ops),
+with whole grids and with split ones (partials and merges in the graph), the
+fused QK RMSNorm + RoPE
 forward and backward (torch.ops.async_op) and the fused q/k/v projection
 kernel (harp_amd.qkv) are recorded once into a
 torch.cuda.CUDAGraph on static tensors and replayed on new inputs.  No
@@ -15,6 +17,7 @@ import torch
 
 import harp_amd
 from harp_amd import _lib
+from tests.gpu_harness import split_plan
 
 pytestmark = pytest.mark.gpu
 
@@ -40,42 +43,73 @@ def _ring_step(q, k, v, do, N, out, m, l, dq, dk, dv):
     ops.ring_attention_backward(q, dq, k, dk, v, dv, do, m, l, D, N, scale)
 
 
-@pytest.mark.parametrize("D", [64, 128])  # compiled kernels; the hand-scheduled D = 128 loops
-def test_ring_attention_graph_replays_equal_eager(D):
-    harp_amd.load_ops()
-    _lib.timing_enable(False)  # no per-launch timing events inside the capture
-    N = 2
-    q, k, v, do = _inputs(0, D=D)
-    out = torch.empty(q.shape, dtype=torch.float32, device=DEV)
-    B, H, T, _ = q.shape
-    m = torch.empty((B, H, T, 1), dtype=torch.bfloat16, device=DEV)
-    l = torch.empty((B, H, T, 1), dtype=torch.float32, device=DEV)
-    dq, dk, dv = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
-    outs = (out, m, l, dq, dk, dv)
+def _one_call_step(q, k, v, do, N):
+    """The one-call operators, which allocate outputs and workspace themselves."""
+    ops = torch.ops.ring_attention_ops
+    scale = 1.0 / math.sqrt(q.size(-1))
+    o, out, m, l = ops.ring_attention_attend(q, k, v, N, scale)
+    return (o, out, m, l, *ops.ring_attention_grad(do, q, k, v, out, m, l, N, scale))
 
+
+def _capture(step):
     side = torch.cuda.Stream()
     side.wait_stream(torch.cuda.current_stream())
     with torch.cuda.stream(side):  # warm-up outside capture, as torch requires
-        _ring_step(q, k, v, do, N, *outs)
+        step()
     torch.cuda.current_stream().wait_stream(side)
     torch.cuda.synchronize()
-
     graph = torch.cuda.CUDAGraph()
     with torch.cuda.graph(graph):
-        _ring_step(q, k, v, do, N, *outs)
+        static = step()
+    return graph, static
 
+
+# (H, T, chunks): whole grids; key pieces in forward and dQ and query splits in
+# dK/dV, whose partials take the dQ partials' place in the workspace; the same
+# of one chunk (the one-call operators' forward)
+SHAPES = pytest.mark.parametrize("H,T,N,whole", [(2, 256, 2, True), (3, 1000, 2, False), (3, 1000, 1, False)])
+HEAD_DIMS = pytest.mark.parametrize("D", [64, 128])  # compiled kernels; the hand-scheduled D = 128 loops
+
+
+@SHAPES
+@HEAD_DIMS
+@pytest.mark.parametrize("one_call", [False, True])
+def test_ring_attention_graph_replays_equal_eager(D, H, T, N, whole, one_call):
+    harp_amd.load_ops()
+    _lib.timing_enable(False)  # no per-launch timing events inside the capture
+    plan = split_plan(1, H, T, D, N, T)
+    assert plan == (1, 1, 1) if whole else min(plan[:2]) > N and plan[2] > 1
+    q, k, v, do = _inputs(0, H=H, T=T, D=D, N=N)
+    if one_call:
+        names = ("o", "out", "m", "l", "dq", "dk", "dv")
+
+        def step(q, k, v, do, outs):
+            return _one_call_step(q, k, v, do, N)
+
+        outs = None
+    else:
+        names = ("out", "m", "l", "dq", "dk", "dv")
+        out = torch.empty(q.shape, dtype=torch.float32, device=DEV)
+        m = torch.empty((1, H, T, 1), dtype=torch.bfloat16, device=DEV)
+        l = torch.empty((1, H, T, 1), dtype=torch.float32, device=DEV)
+        outs = (out, m, l, torch.empty_like(q), torch.empty_like(k), torch.empty_like(v))
+
+        def step(q, k, v, do, outs):
+            _ring_step(q, k, v, do, N, *outs)
+            return outs
+
+    graph, static = _capture(lambda: step(q, k, v, do, outs))
     for seed in (1, 2, 3):
-        nq, nk, nv, ndo = _inputs(seed, D=D)
+        nq, nk, nv, ndo = _inputs(seed, H=H, T=T, D=D, N=N)
         for dst, src in ((q, nq), (k, nk), (v, nv), (do, ndo)):
             dst.copy_(src)
         graph.replay()
         torch.cuda.synchronize()
-        got = [t.clone() for t in outs]
+        got = [t.clone() for t in static]
         # eager on the same inputs, into fresh tensors
-        ref = [torch.empty_like(t) for t in outs]
-        _ring_step(nq, nk, nv, ndo, N, *ref)
+        ref = step(nq, nk, nv, ndo, outs and [torch.empty_like(t) for t in outs])
         torch.cuda.synchronize()
-        for name, a, b in zip(("out", "m", "l", "dq", "dk", "dv"), got, ref):
+        for name, a, b in zip(names, got, ref):
             assert torch.equal(a, b), (seed, name)
 
 

@@ -17,7 +17,7 @@ import pytest
 import torch
 
 from oracle import ring_attn_oracle as orc
-from tests.gpu_harness import run_hip
+from tests.gpu_harness import run_hip, split_plan
 from tests.parity import TOL_GRAD, TOL_LSE, TOL_O, rel_fro, rel_max
 from tests.test_golden import case_tensors, load_cases
 
@@ -195,19 +195,24 @@ def test_config5_ragged_masked():
 
 # --- boundary semantics ----------------------------------------------------------
 
-def _small(D=64):
-    q, ks, vs, do = orc.make_inputs(1, 4, 200, D, 3, seed=0, chunk_len=136)
+def _small(D=64, chunk=136):
+    """One query tile of four heads: 136-key chunks run whole, 700-key ones
+    split their ring steps' keys (forward and dQ)."""
+    assert (min(split_plan(1, 4, 200, D, 3, chunk)[:2]) > 3) == (chunk > 136)
+    q, ks, vs, do = orc.make_inputs(1, 4, 200, D, 3, seed=0, chunk_len=chunk)
     return q, ks, vs, do, 1.0 / math.sqrt(D)
 
 
 # D = 64 runs the compiled kernels, D = 72 the compiled kernels with their
 # 16-wide d tail, D = 128 the hand-scheduled loops
 SMALL_DIMS = pytest.mark.parametrize("D", [64, 72, 128])
+SMALL_CHUNKS = pytest.mark.parametrize("chunk", [136, 700])
 
 
+@SMALL_CHUNKS
 @SMALL_DIMS
-def test_layouts_dtypes_and_paths_agree(D):
-    q, ks, vs, do, scale = _small(D)
+def test_layouts_dtypes_and_paths_agree(D, chunk):
+    q, ks, vs, do, scale = _small(D, chunk)
     base = run_hip(q, ks, vs, do, scale)
     ref = _oracle_full(q, ks, vs, do, scale)
     _check_all(base, ref)
@@ -236,13 +241,14 @@ def test_layouts_dtypes_and_paths_agree(D):
                 assert same, (kw, key)
 
 
+@SMALL_CHUNKS
 @SMALL_DIMS
 @pytest.mark.parametrize("rank", [1, 2])
-def test_ring_rank_order(rank, D):
+def test_ring_rank_order(rank, D, chunk):
     """ring_rank changes the chunk visiting order; the result stays within the
     bar of the oracle, and differs from rank 0 only by bf16 rounding of P
     (the running max, the reference point of P, is reached in another order)."""
-    q, ks, vs, do, scale = _small(D)
+    q, ks, vs, do, scale = _small(D, chunk)
     ref = _oracle_full(q, ks, vs, do, scale, rank=rank)
     base = run_hip(q, ks, vs, do, scale)
     r = run_hip(q, ks, vs, do, scale, ring_rank=rank)
@@ -252,9 +258,10 @@ def test_ring_rank_order(rank, D):
     assert err_o < 5e-3 and err_lse < 1e-4, (err_o, err_lse)
 
 
+@SMALL_CHUNKS
 @SMALL_DIMS
-def test_bf16_m_is_lse_consistent(D):
-    q, ks, vs, do, scale = _small(D)
+def test_bf16_m_is_lse_consistent(D, chunk):
+    q, ks, vs, do, scale = _small(D, chunk)
     r16 = run_hip(q, ks, vs, do, scale, backward=False)
     r32 = run_hip(q, ks, vs, do, scale, m_dtype=torch.float32, backward=False)
     assert torch.equal(r16["m"].float(), r16["m"].float().bfloat16().float())
@@ -276,9 +283,10 @@ def test_sixteen_chunks_split_sixteen_ways(D):
     forward and dQ split the ring steps 16 ways, so both merges take their
     path for more than eight splits (the maximum over every split's m first,
     then two groups of eight).  Ragged and empty chunks, ring rank 5."""
-    lens = [40, 0, 33, 40, 1, 40, 0, 17, 40, 40, 29, 0, 40, 8, 40, 40]
+    lens = [200, 0, 133, 200, 1, 200, 0, 97, 200, 200, 129, 0, 200, 8, 200, 200]
+    assert split_plan(1, 1, 100, D, 16, 200, lens) == (16, 16, 1)
     print(f"[16 chunks D={D}]", flush=True)
-    q, ks, vs, do = orc.make_inputs(1, 1, 100, D, len(lens), seed=16, chunk_len=40)
+    q, ks, vs, do = orc.make_inputs(1, 1, 100, D, len(lens), seed=16, chunk_len=200)
     scale = 1.0 / math.sqrt(D)
     res = run_hip(q, ks, vs, do, scale, ring_rank=5, kv_lens=lens)
     ref = _oracle_full(q, ks, vs, do, scale, rank=5, lens=lens)
@@ -287,7 +295,8 @@ def test_sixteen_chunks_split_sixteen_ways(D):
 
 @pytest.mark.parametrize("D", [64, 128])  # compiled kernels; the hand-scheduled D = 128 loops
 @pytest.mark.parametrize("via", ["abi", "ops"])
-def test_very_negative_lse_with_pad_keys(via, D):
+@pytest.mark.parametrize("lens", [[100, 70], [900, 700]])  # whole; keys split, pieces without a valid key
+def test_very_negative_lse_with_pad_keys(via, D, lens):
     """Rows whose every score is far below -88 (LSE about -120), with ragged
     chunks, so pad keys (zero K / V rows, score 0) sit in the tail tiles.  A
     pad key's P = exp(0 - LSE) would overflow; the backward must still give
@@ -297,8 +306,8 @@ def test_very_negative_lse_with_pad_keys(via, D):
     # can resolve to the bar (emulating bf16 dS alone costs 3.5e-2 there, and
     # 2e-3 here).
     g = torch.Generator().manual_seed(11)
-    B, H, T, N, tc = 1, 2, 40, 2, 100
-    lens = [100, 70]
+    B, H, T, N, tc = 1, 2, 40, 2, lens[0]
+    assert (min(split_plan(B, H, T, D, N, tc, lens)[:2]) > N) == (tc > 100)
     u = torch.randn((1, H, 1, D), generator=g)
     q = (-20.0 * u + 0.5 * torch.randn((B, H, T, D), generator=g)).to(torch.bfloat16)
     ks = [(u + torch.randn((B, H, tc, D), generator=g)).to(torch.bfloat16) for _ in range(N)]
@@ -313,9 +322,10 @@ def test_very_negative_lse_with_pad_keys(via, D):
     _check_all(res, ref)
 
 
+@SMALL_CHUNKS
 @SMALL_DIMS
-def test_nan_propagates_to_its_row_only(D):
-    q, ks, vs, do, scale = _small(D)
+def test_nan_propagates_to_its_row_only(D, chunk):
+    q, ks, vs, do, scale = _small(D, chunk)
     q = q.clone()
     q[0, 1, 7, 3] = float("nan")
     res = run_hip(q, ks, vs, do, scale, backward=False)

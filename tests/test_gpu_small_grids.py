@@ -10,6 +10,7 @@ import torch
 
 import harp_amd
 from harp_amd import ops as H_ops
+from tests.gpu_harness import split_plan
 
 pytestmark = pytest.mark.gpu
 
@@ -41,6 +42,8 @@ def _rel(a, b):
 @pytest.mark.parametrize("B,H,T,D,sp,chunk,lens,rank", SHAPES)
 @pytest.mark.parametrize("grads", ["bf16", "fp32", "bf16 unaligned"])
 def test_split_calls_against_fp64(B, H, T, D, sp, chunk, lens, rank, grads):
+    _, dq_splits, dkdv_splits = split_plan(B, H, T, D, sp, chunk, lens)
+    assert dq_splits > sp and (dkdv_splits > 1) == (T >= 576)  # 513 queries: two splits don't pay
     if grads == "bf16 unaligned" and D == 128:
         pytest.skip("head dim 128 stores bf16 gradients 8 bytes at a time: the C ABI refuses such views")
     g = torch.Generator(device=DEV).manual_seed(T + D)
@@ -165,6 +168,7 @@ def test_one_call_operators_on_small_grids(B, H, T, D, sp, chunk, lens, rank):
     the merge, D formed by each key piece's dQ block."""
     harp_amd.load_ops()
     ops = torch.ops.ring_attention_ops
+    assert (split_plan(B, H, T, D, sp, chunk, lens)[0] > sp) == (T != 2049)  # 2049: 770 keys a tile don't pay
     g = torch.Generator(device=DEV).manual_seed(T + D)
     q, dout = (torch.randn(B, T, H, D, device=DEV, generator=g).to(torch.bfloat16).transpose(1, 2) for _ in range(2))
     k, v = (torch.randn(B, sp * chunk, H, D, device=DEV, generator=g).to(torch.bfloat16).transpose(1, 2) for _ in range(2))

@@ -33,7 +33,7 @@
 //   k-tile = 64 elements: x tile 256 x 64 and W tile 256 x 64 (32 KB each),
 //            copied global -> LDS by buffer_load ... lds into two stages.
 // These blocks are MFMA- and LDS-bound and the fastest per token once the CUs
-// are full (386 us, 1200 TFLOP/s, at 8192 tokens x 24 heads x 3).  Two smaller
+// are full (393 us, 1180 TFLOP/s, at 8192 tokens x 24 heads x 3).  Two smaller
 // ones, bit for bit the same arithmetic, serve grids that leave CUs idle and
 // the last round of the CUs; there a tile's few MFMAs don't cover the memory's
 // latency with one tile of lead, so more stages are in flight:
@@ -42,7 +42,7 @@
 //   32 tokens per wave, 1 head: 4 waves, 128 tokens x 1 head, 32 KB a tile,
 //            four stages.  At 256 tokens x 30 heads it fills 180 of the CUs
 //            where the large blocks fill 45, and reads the 88 MB of weights at
-//            2.5 TB/s: 83 -> 35 us.
+//            2.6 TB/s: 83 -> 34 us.
 // launch_proj has the rule.
 // Pipeline: one barrier per tile, in its last k-step, after which nobody
 // reads tile t's stage any more (its last fragments are in registers) and

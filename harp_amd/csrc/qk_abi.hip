@@ -171,8 +171,9 @@ int resolve_workspace(void** ws, size_t* ws_bytes, size_t need, hipStream_t stre
 }
 
 // Scratch of the allocation-free backward (harp_qk_norm_rope_backward_noalloc):
-// the weight-gradient partials of at most kQkBwdMaxBlocks row blocks plus their
-// group sums, for any D <= 256: (2048 + 32) x 256 floats = 2.03 MiB, held by
+// the weight-gradient partials at the size of the largest workspace, for any
+// D <= 256: (2048 + 32) x 256 floats = 2.03 MiB (of which the kernels write at
+// most kQkBwdMaxLaunch rows), held by
 // every device the library runs on until the process ends.  In host code the
 // name is only a stand-in; kernels get the device address that
 // hipGetSymbolAddress returns for the current device (scratch_ptr below).

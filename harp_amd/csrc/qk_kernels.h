@@ -54,14 +54,16 @@ struct QkBwdParams {
   float* wpart;        // [blocks][D] fp32 weight-gradient partials (workspace)
 };
 
-// The weight-gradient workspace (harp_qk_backward_workspace_bytes): one
-// partial row of D floats for each of up to kQkBwdMaxBlocks 16-row blocks,
-// and one row more per kWgGroupRows of them.
+// The size of the weight-gradient workspace (harp_qk_backward_workspace_bytes):
+// a row of D floats for each of up to kQkBwdMaxBlocks 16-row blocks, and one
+// more per kWgGroupRows of them.  It is what callers have always been asked
+// for; the kernels write only the first bwd_launch_blocks rows, at most
+// kQkBwdMaxLaunch.
 constexpr int kQkBwdMaxBlocks = 2048;
 int bwd_blocks(const QkShape& sh);
 constexpr int kWgGroupRows = 64;
-// Blocks the backward kernel is launched with (each a contiguous range of
-// rows, one partial row), never more than bwd_blocks.
+// Blocks the backward kernel is launched with (one partial row each; every
+// stride-th step of its XCD's range of rows), never more than bwd_blocks.
 // (1024: four 4-wave blocks per CU; the forward's registers fit eight)
 constexpr int kQkBwdMaxLaunch = 1024;
 constexpr int kQkFwdMaxLaunch = 2048;

@@ -32,12 +32,13 @@
 // RMSNorm row's loads, sum, square root and division are one serial chain, so
 // the kernels with RMSNorm walk their rows with the next loads in flight, and
 // the forward takes two heads of a token at once (one RoPE row, one root and
-// division for both).  Buffers cycled through 800 MB, one row group per block
-// without a prefetch -> this, at [B,H,S,D]: [1,24,8192,128] forward 28.2 ->
-// 23.5 us, backward 47.5 -> 36.5 (4.1 TB/s; a 4 GiB copy reaches 4.9);
-// [1,30,16384,128] 63 -> 54 and 105 -> 82; [2,16,8192,64] 28 -> 17 and 50 -> 26
-// (16 lanes per row left half of them idle); [1,30,256,128] 8 and 13.1 -> 10.2
-// (one reduction launch fewer).
+// division for both).  Calls back to back over buffers cycled through 800 MB,
+// one row group per block without a prefetch -> this, at [B,H,S,D]:
+// [1,24,8192,128] forward 26.7 -> 22.8 us, backward with its reduction 42.1 ->
+// 31.4 (5.0 TB/s, the rate of a large copy); [1,30,16384,128] 59.1 -> 53.2 and
+// 104.8 -> 80.5; [2,16,8192,64] 31.0 -> 17.5 and 48.4 -> 24.2 (16 lanes per row
+// left half of them idle); [1,30,256,128] backward 12.6 -> 9.7 (one reduction
+// launch fewer).
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -448,10 +449,12 @@ __global__ __launch_bounds__(256) void rope_kernel(RopeParams p) {
 // (truncated, like the reference's other bf16 stores).  A launch behind
 // another costs about 4.5 us here whatever it does: with at most
 // kQkBwdMaxLaunch rows one launch ends sooner than two levels of 64-row groups
-// did (13.1 -> 10.2 us for the whole backward at 30 heads x 256 rows).  Block x sums columns
-// 8x .. 8x + 7 with 128 row lanes, each taking every 128th row (at most
-// kQkBwdMaxLaunch / 128 independent loads in flight per thread), and LDS adds
-// the lane sums in order.
+// did (12.6 -> 9.7 us for the whole backward at 30 heads x 256 rows).  Block x
+// sums columns 8x .. 8x + 7 with 128 row lanes, each taking every 128th row (at
+// most kQkBwdMaxLaunch / 128 independent loads in flight per thread), and LDS
+// adds the lane sums in order.  (The order, and so the last bit, of a weight
+// gradient depends on the number of partial rows; y, rms and dx depend on
+// neither the grid nor the lanes per row.)
 constexpr int kWgCols = 8, kWgLanes = 128;
 __global__ __launch_bounds__(kWgCols* kWgLanes) void wgrad_sum_kernel(const float* src, int nrows, int D, void* dst,
                                                                       int dst_f32) {

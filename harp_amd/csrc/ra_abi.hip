@@ -182,7 +182,8 @@ int device_cus() {
 // kMergeUs is the launch's cost on the host, which bounds calls this small: 8
 // heads x 512 x 512 at head dim 64, forward + backward through autograd, took
 // 94 us whole and 105 with its three grids split in two, although their GPU
-// time fell from 48 to 45.
+// time fell from 48 to 45.  (A replayed graph does not pay that part; the rule
+// does not tell captured calls apart.)
 constexpr double kFwdUsPerKey = 0.028, kDqUsPerKey = 0.035, kDkdvUsPerQuery = 0.045;
 constexpr double kMergeUs = 10., kMergeBytesPerUs = 5e6;
 // fewer keys or queries than this per block are all fixed cost
@@ -206,8 +207,8 @@ double split_cost(double us, int64_t part, int n, double bytes) {
 // keys, in `pieces` runs of `piece` keys (a multiple of 128, the longest key
 // tile).  30 heads x 1024 queries x 1024 keys of one chunk stay whole (two
 // pieces: 33.2 us against 32.0); 8 heads x 1500 x 1500 take four pieces, the
-// forward 38.8 -> 32.8 us at head dim 128 and 30 -> 22 at 64; 8 heads x 4096 x
-// 4096 two, 95 -> 80.
+// forward 39.8 -> 33.2 us at head dim 128 and 30.6 -> 23.0 at 64; 8 heads x
+// 4096 x 4096 two, 93 -> 76.
 struct KvPlan {
   int n_split;
   int pieces;  // per chunk
@@ -270,8 +271,8 @@ void fill_kv_table(ChunkTable* ct, const KvPlan& kp, const Geometry& g, const vo
 }
 
 // Query splits of the dK/dV kernel (with dQ's key pieces: backward of 8 heads x
-// 1500 x 1500 111 -> 82 us at head dim 128, 74 -> 53 at 64; x 4096 x 4096 268
-// -> 241).
+// 1500 x 1500 112 -> 79 us at head dim 128, 75 -> 53 at 64; x 4096 x 4096 268
+// -> 230).
 struct QPlan {
   int n_split;
   int rows;  // queries per split, a multiple of 64

@@ -1,7 +1,7 @@
 """Python call pattern of the ring-attention block on the HIP path.
 
 * :class:`RingAttention` mirrors ``CPURingAttention``
-  (src/models/z_image/module/attn.py:15-49): same arguments, same caller-
+  (src/models/z_image/module/attn.py:15-49): same arguments, same
   ``out`` (fp32, q's token-major strides), bf16 ``m_i`` and fp32 ``l_i``, same
   saved tensors, same ``D = rowsum(dO * O)``.  Each direction is one operator
   call (``ring_attention_attend``, ``ring_attention_grad`` of
@@ -48,8 +48,9 @@ class RingAttention(torch.autograd.Function):
         ctx.scale = scale
         # attn.py:24-32: out, m_i and l_i are allocated, filled and out is cast
         # to q's dtype; the operator allocates them in the same layouts and its
-        # kernel stores both forms of out.  Without a gradient to take, the
-        # fp32 one is neither stored nor kept.
+        # kernel stores both forms of out.  Where no input requires a gradient,
+        # the fp32 one is neither stored nor kept (needs_input_grad follows
+        # requires_grad, also under no_grad).
         keep = any(ctx.needs_input_grad)
         o, out, m_i, l_i = _ops().ring_attention_attend(local_q, local_k, local_v, sp_size, scale, ring_rank, kv_lens,
                                                         ctx.chunk_len, keep)

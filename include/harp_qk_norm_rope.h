@@ -150,9 +150,9 @@ HARP_QK_API int harp_qk_norm_rope_backward_noalloc(const void* dy, const int64_t
                                                    int s_len, int h_len, void* stream);
 
 /* Device workspace the two backward entry points with RMSNorm need
- * ((size_t)-1 when the arguments are invalid): the weight-gradient partial
- * sums of up to 2048 row blocks and their 64-row group sums, at most
- * (2048 + 32) x h_len floats. */
+ * ((size_t)-1 when the arguments are invalid), for the weight-gradient partial
+ * sums: a row of h_len floats per 16 rows of x, at most 2048, and one more per
+ * 64 of those (at most (2048 + 32) x h_len floats).  Not all of it is written. */
 HARP_QK_API size_t harp_qk_backward_workspace_bytes(int batch, int h_num, int s_len, int h_len);
 
 /*

@@ -57,8 +57,8 @@ def _bits(t):
 
 @pytest.mark.parametrize("gw_dtype", [torch.float32, torch.bfloat16])
 def test_noalloc_backward_equals_workspace_backward(gw_dtype):
-    # first call: 2048 row blocks (the scratch's maximum) at D = 128; second:
-    # a smaller problem at another D, which reads fewer partial rows
+    # first call: 1024 partial rows (the most the backward kernel is launched
+    # with) at D = 128; second: a smaller problem at another D, which reads fewer
     for (B, H, S, D), seed in (((1, 24, 8192, 128), 1), ((2, 3, 100, 72), 2)):
         print(f"[noalloc backward B={B} H={H} S={S} D={D} grad_weight {gw_dtype}]", flush=True)
         args = _inputs(B, H, S, D, seed)
